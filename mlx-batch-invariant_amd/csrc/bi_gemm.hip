@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 #include "bi_gemm_kernel.h"
 
 namespace {
@@ -24,11 +26,11 @@ constexpr Geometry kGeometries[] = {BI_GEOMETRIES(BI_GEO_ENTRY)};
 #undef BI_GEO_ENTRY
 constexpr int kNumGeometries = sizeof(kGeometries) / sizeof(kGeometries[0]);
 
-KernelFn select_kernel(int dtype, int trans_b, int g) {
+KernelFn select_kernel(int dtype, int trans_b, int g, bool ragged) {
   switch (dtype) {
-    case BI_F32: return bi_gemm_kernel_f32(g, trans_b != 0);
-    case BI_F16: return bi_gemm_kernel_f16(g, trans_b != 0);
-    case BI_BF16: return bi_gemm_kernel_bf16(g, trans_b != 0);
+    case BI_F32: return bi_gemm_kernel_f32(g, trans_b != 0, ragged);
+    case BI_F16: return bi_gemm_kernel_f16(g, trans_b != 0, ragged);
+    case BI_BF16: return bi_gemm_kernel_bf16(g, trans_b != 0, ragged);
   }
   return nullptr;
 }
@@ -201,15 +203,53 @@ VecFlags vec_flags(const void* a, const void* b, int64_t N, int64_t K, int dtype
   return v;
 }
 
-// The geometry bi_gemm launches: pick_geometry's, unless that one takes
-// aligned operands only and these are not; then the 128 x 128 footprint.
-int pick_for(const void* a, const void* b, int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
-  int g = pick_geometry(M, N, dtype, trans_b);
-  if (kGeometries[g].pl) {
-    const VecFlags v = vec_flags(a, b, N, K, dtype, trans_b, kGeometries[g]);
-    if (!(v.a && v.b)) g = 3;
+// Geometry for operands that are not 16-byte aligned (the register-staged
+// kernels): the least estimated time per element of K, from a grid of every
+// footprint that has such a kernel over M = 1..1024, K = 501..4095 and N =
+// 601..5001 (both layouts, bf16 and fp32; every size odd). A 64 x 32, 64 x 64
+// or 128 x 128 tile costs a round of the CUs each time its tiles pass a
+// multiple of them (N = 4097, M = 1024: 264 tiles of 128 x 128 take 95 us, 240
+// at N = 5001, M = 700, K = 2047 30 us); the small tiles run several
+// workgroups a CU: their time is flat for few tiles, grows to `one` as the
+// tiles reach one a CU, and by `more` for each further 256. Units: 0.1 us per
+// 1000 elements of K.
+int pick_ragged(int64_t M, int64_t N, int dtype, int trans_b) {
+  struct Cost { int flat, one, more; };  // one == 0: whole rounds of `flat`
+  const bool f32 = dtype == BI_F32;
+  const Cost g0 = f32 ? Cost{44, 56, 39} : trans_b ? Cost{20, 27, 18} : Cost{30, 52, 34};
+  const Cost g1 = f32 ? Cost{65, 95, 68} : trans_b ? Cost{34, 59, 35} : Cost{42, 86, 48};
+  const Cost g2 = {f32 ? 190 : 62, 0, 0};
+  const Cost g3 = {f32 ? 650 : 108, 0, 0};
+  const Cost g5 = {f32 ? (M <= 16 ? 63 : 100) : 44, 0, 0};
+  struct Cand { int g, bm, bn; Cost c; };
+  const Cand cands[] = {{0, 16, 16, g0}, {1, 64, 16, g1}, {5, 64, 32, g5}, {2, 64, 64, g2},
+                        {3, 128, 128, g3}};
+  int best = 0;
+  int64_t best_cost = -1;
+  for (const Cand& k : cands) {
+    const int64_t tiles = ceil_div(M, k.bm) * ceil_div(N, k.bn);
+    int64_t cost;
+    if (k.c.one) {
+      cost = k.c.flat;
+      cost = std::max(cost, k.c.one * std::min(tiles, (int64_t)256) / 256);
+      cost = std::max(cost, k.c.more * tiles / 256);
+    } else {
+      cost = ceil_div(tiles, 256) * k.c.flat;
+    }
+    if (best_cost < 0 || cost < best_cost) {
+      best = k.g;
+      best_cost = cost;
+    }
   }
-  return g;
+  return best;
+}
+
+// The geometry bi_gemm launches: pick_geometry's for operands whose every
+// row may be read as aligned 16-byte vectors by it, else pick_ragged's.
+int pick_for(const void* a, const void* b, int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
+  const int g = pick_geometry(M, N, dtype, trans_b);
+  const VecFlags v = vec_flags(a, b, N, K, dtype, trans_b, kGeometries[g]);
+  return v.a && v.b ? g : pick_ragged(M, N, dtype, trans_b);
 }
 
 // start/stop (optional): hipEvents that receive the dispatch's own start and
@@ -234,11 +274,9 @@ int launch(const void* a, const void* b, const void* bias, void* out, int64_t M,
   const VecFlags v = vec_flags(a, b, N, K, dtype, trans_b, G);
   if (G.pl && !(v.a && v.b))
     return bi::fail(BI_EUNSUPPORTED, "bi_gemm: geometry %d takes 16-byte aligned operands only", g);
-  p.vec_a = v.a;
-  p.vec_b = v.b;
   const int64_t blocks = (int64_t)p.tiles_m * p.tiles_n;
   if (blocks > INT32_MAX) return bi::fail(BI_EINVAL, "bi_gemm: too many tiles");
-  KernelFn fn = select_kernel(dtype, trans_b, g);
+  KernelFn fn = select_kernel(dtype, trans_b, g, !(v.a && v.b));
   if (!fn) return bi::fail(BI_EUNSUPPORTED, "bi_gemm: geometry %d not built for this dtype", g);
   if (start || stop)
     hipExtLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(64 * G.waves), 0,
@@ -459,8 +497,6 @@ int qlaunch(const void* x, const void* w, const void* scales, const void* biases
   p.tiles_n = (int)ceil_div(N, G.bn);
   p.alpha = 1.f;
   p.beta = 1.f;
-  p.vec_a = 1;
-  p.vec_b = 1;
   p.qs = scales;
   p.qz = biases;
   p.qgroup_shift = group_shift(group_size);

@@ -60,7 +60,6 @@ struct GemmArgs {
   int64_t M, N, K;
   int tiles_m, tiles_n;
   float alpha, beta;
-  int vec_a, vec_b;  // rows of A / rows of B may be read as aligned 16-byte vectors
   // Affine-quantized B (quantized kernels only): B is the packed (N, K * bits
   // / 32) uint32 weight, qs / qz the (N, K / group) scales and biases in the
   // element type, group = 1 << qgroup_shift.
@@ -224,23 +223,55 @@ __device__ inline void tile_coords(int tile, int tiles_m, int tiles_n, int& mi, 
   ni = within / rows;
 }
 
-// 16-byte chunk of row `row` of a row-major matrix with leading dimension
-// `ld`, starting at element k, read element by element; elements of rows at
-// or past `rows` or at or past column `limit` are zero. The path for operands
-// the buffer path cannot take (unaligned, or panels of 2 GiB and more).
+// 16 bytes from an address with the element type's alignment only: one
+// global_load_dwordx4 (the target allows unaligned vector loads).
 template <typename T>
-__device__ inline uint4 load_chunk(const T* __restrict__ base, int64_t row, int64_t rows,
-                                   int64_t ld, int64_t k, int64_t limit) {
-  constexpr int E = 16 / sizeof(T);
-  const bool row_ok = row < rows;
-  union {
-    uint4 u;
-    T e[E];
-  } r;
-  const T* p = base + (row_ok ? row : 0) * ld;
+__device__ __forceinline__ uint4 load_any(const T* p) {
+  u32x4_t v;
+  __builtin_memcpy(&v, p, 16);
+  return __builtin_bit_cast(uint4, v);
+}
+
+// The 16-byte chunk that starts at element f of an array of `total`
+// elements, its first `valid` elements (all inside the array) kept and the
+// others zero; valid <= 0 gives zeros. A chunk that would run past the array
+// is read from the array's last 16 bytes and shifted.
+template <typename T>
+__device__ inline uint4 tail_chunk(const T* base, int64_t f, int64_t total, int64_t valid) {
+  constexpr int E = 16 / sizeof(T), W = 8 * sizeof(T);  // elements per chunk, bits per element
+  using Bits = typename std::conditional<sizeof(T) == 2, uint16_t, uint32_t>::type;
+  if (valid <= 0) return make_uint4(0, 0, 0, 0);
+  const int keep = valid < E ? (int)valid : E;
+  uint64_t lo = 0, hi = 0;
+  if (total >= E) {
+    const int64_t at = f < total - E ? f : total - E;
+    const uint4 v = load_any<T>(base + at);
+    lo = ((uint64_t)v.y << 32) | v.x;
+    hi = ((uint64_t)v.w << 32) | v.z;
+    int drop = (int)(f - at) * W;  // drop + keep * W <= 128
+    if (drop >= 64) {
+      lo = hi;
+      hi = 0;
+      drop -= 64;
+    }
+    if (drop) {
+      lo = (lo >> drop) | (hi << (64 - drop));
+      hi >>= drop;
+    }
+  } else {
 #pragma unroll
-  for (int i = 0; i < E; i++) r.e[i] = (row_ok && k + i < limit) ? p[k + i] : T(0);
-  return r.u;
+    for (int i = 0; i < E; i++) {
+      if (i < keep) {
+        const uint64_t e = __builtin_bit_cast(Bits, base[f + i]);
+        if (i < E / 2) lo |= e << (W * i);
+        else hi |= e << (W * (i - E / 2));
+      }
+    }
+  }
+  const int bits = keep * W;
+  if (bits < 64) lo &= ((uint64_t)1 << bits) - 1;
+  hi &= bits <= 64 ? 0 : ~(uint64_t)0 >> (128 - bits);
+  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
 }
 
 // Raw buffer resources (CDNA "V#"): loads whose byte offset is at or past
@@ -339,8 +370,6 @@ struct GemmTile {
   static constexpr int FM = WTM / 16, FN = WTN / 16;  // 16x16 MFMA blocks per wave
   static constexpr int A_CH = BM * RC;                // chunks per stage
   static constexpr int B_CH = BN * RC;
-  static constexpr int LA = (A_CH + NT - 1) / NT;     // chunks per thread per stage (VGPR path)
-  static constexpr int LB = (B_CH + NT - 1) / NT;
   static constexpr int NN_CPR = BN * (int)sizeof(T) / 16;  // chunks per k-row, (K, N) B tile
   static constexpr int STAGE_CH = A_CH + B_CH;
   static constexpr int LDW = PL ? NW - WM * WN : NW;  // waves that issue loads
@@ -448,48 +477,101 @@ struct GemmTile {
     }
   }
 
-  // Register-staged loads for operands the buffer path cannot take.
-  __device__ __forceinline__ void gload_slow(int64_t s, uint4* ra, uint4* rb) const {
-    const int64_t k0 = s * EPS;
+  // ---- Register-staged path (RG kernels): operands the buffer path cannot
+  // take, i.e. rows that are not 16-byte aligned, or panels of 2 GiB and more.
+  // Rows past M (columns past N of an (N, K) B) read the last one, and a
+  // (K, N) chunk past N reads on into the next rows: what they produce lies
+  // outside C and is never stored. Stages that lie wholly below kfull() read
+  // inside the operands with plain 16-byte loads; the rest go through
+  // tail_chunk, which zeroes elements past K. The waves that do not compute,
+  // where there are such, load and stage every operand, so a stage is written
+  // while the one before it is computed. Bound by those loads: an access that
+  // is not 16-byte aligned takes the address unit about 64 cycles a wave
+  // instead of 16 (any smaller alignment alike), 0.5 us per 32 KB stage.
+  // Against one element per load and two barriers a stage (bf16): M = 301,
+  // K = 1001, N = 3001 (K, N) 43.2 -> 13.7 us; M = 2048, K = 4095, N = 4096
+  // (N, K) 938 -> 134 us; M = 1 55 -> 10.8 us.
+  static constexpr int RNT = NW > CW ? 64 * (NW - CW) : NT;  // loading threads
+  static constexpr int RLA = (A_CH + RNT - 1) / RNT, RLB = (B_CH + RNT - 1) / RNT;
+  static constexpr int RGP = RLA + RLB > 4 ? 2 : 4;  // stages of loads in flight (registers)
+  struct RStage {
+    uint4 a[RLA], b[RLB];
+  };
+  const T* rg_a[RLA];
+  const T* rg_b[RLB];
+  int rtid;  // index among the loading threads
+
+  // K elements of which every chunk, also one that runs past N, ends inside B.
+  __device__ __forceinline__ int64_t kfull() const {
+    if constexpr (TB) return K;
+    return K - (EPC - 1 + N - 1) / N;
+  }
+
+  __device__ __forceinline__ void init_ragged() {
+    rtid = tid - (NT - RNT);
 #pragma unroll
-    for (int i = 0; i < LA; i++) {
-      const int q = tid + i * NT;
-      if (A_CH % NT == 0 || q < A_CH)
-        ra[i] = load_chunk<T>(A, m0 + q / RC, M, K, k0 + (q % RC) * EPC, K);
+    for (int i = 0; i < RLA; i++) {
+      const int q = rtid + i * RNT;
+      rg_a[i] = A + min(m0 + q / RC, M - 1) * K + (q % RC) * EPC;
     }
 #pragma unroll
-    for (int i = 0; i < LB; i++) {
-      const int q = tid + i * NT;
-      if (B_CH % NT == 0 || q < B_CH) {
-        if constexpr (TB)
-          rb[i] = load_chunk<T>(B, n0 + q / RC, N, K, k0 + (q % RC) * EPC, K);
-        else
-          rb[i] = load_chunk<T>(B, k0 + q / NN_CPR, K, N, n0 + (q % NN_CPR) * EPC, N);
+    for (int i = 0; i < RLB; i++) {
+      const int q = rtid + i * RNT;
+      if constexpr (TB)
+        rg_b[i] = B + min(n0 + q / RC, N - 1) * K + (q % RC) * EPC;
+      else  // (the last loads of an uneven split lie past the tile: row 0)
+        rg_b[i] = B + (int64_t)(q < B_CH ? q / NN_CPR : 0) * N + min(n0 + (q % NN_CPR) * EPC, N - 1);
+    }
+  }
+
+  __device__ __forceinline__ void rg_load(int64_t s, RStage& st) const {
+    const int64_t ao = s * EPS, bo = TB ? ao : ao * N;
+#pragma unroll
+    for (int i = 0; i < RLA; i++) st.a[i] = load_any<T>(rg_a[i] + ao);
+#pragma unroll
+    for (int i = 0; i < RLB; i++) st.b[i] = load_any<T>(rg_b[i] + bo);
+  }
+
+  __device__ __forceinline__ void rg_load_tail(int64_t s, RStage& st) const {
+    const int64_t k0 = s * EPS;
+#pragma unroll
+    for (int i = 0; i < RLA; i++) {
+      const int q = rtid + i * RNT;
+      const int64_t r = min(m0 + q / RC, M - 1), k = k0 + (q % RC) * EPC;
+      st.a[i] = tail_chunk<T>(A, r * K + k, M * K, K - k);
+    }
+#pragma unroll
+    for (int i = 0; i < RLB; i++) {
+      const int q = rtid + i * RNT;
+      if constexpr (TB) {
+        const int64_t r = min(n0 + q / RC, N - 1), k = k0 + (q % RC) * EPC;
+        st.b[i] = tail_chunk<T>(B, r * K + k, N * K, K - k);
+      } else {
+        const int64_t k = k0 + q / NN_CPR, n = n0 + (q % NN_CPR) * EPC;
+        st.b[i] = tail_chunk<T>(B, k * N + n, K * N, k < K ? N - n : 0);
       }
     }
   }
 
-  __device__ __forceinline__ void sstore(Slot sl, const uint4* ra, const uint4* rb) const {
-    uint4* As = sl.a;
-    uint4* Bs = sl.b;
+  __device__ __forceinline__ void rg_store(Slot sl, const RStage& st) const {
 #pragma unroll
-    for (int i = 0; i < LA; i++) {
-      const int q = tid + i * NT;
-      if (A_CH % NT == 0 || q < A_CH) {
+    for (int i = 0; i < RLA; i++) {
+      const int q = rtid + i * RNT;
+      if (A_CH % RNT == 0 || q < A_CH) {
         const int r = q / RC, c = q % RC;
-        As[r * RC + (c ^ swz_k<RC>(r))] = ra[i];
+        sl.a[r * RC + (c ^ swz_k<RC>(r))] = st.a[i];
       }
     }
 #pragma unroll
-    for (int i = 0; i < LB; i++) {
-      const int q = tid + i * NT;
-      if (B_CH % NT == 0 || q < B_CH) {
+    for (int i = 0; i < RLB; i++) {
+      const int q = rtid + i * RNT;
+      if (B_CH % RNT == 0 || q < B_CH) {
         if constexpr (TB) {
           const int r = q / RC, c = q % RC;
-          Bs[r * RC + (c ^ swz_k<RC>(r))] = rb[i];
+          sl.b[r * RC + (c ^ swz_k<RC>(r))] = st.b[i];
         } else {
           const int r = q / NN_CPR, c = q % NN_CPR;
-          Bs[r * NN_CPR + (c ^ swz_nn<T, NN_CPR>(r))] = rb[i];
+          sl.b[r * NN_CPR + (c ^ swz_nn<T, NN_CPR>(r))] = st.b[i];
         }
       }
     }
@@ -1263,25 +1345,86 @@ struct GemmTile {
       q_rounds<false, true, GS, NGR>(slots, nst, nsteps, q, acc, P, X);
   }
 
-  // Register-staged path (unaligned operands): two slots, double buffered.
+  // Register-staged path: stage s goes from registers to slot s mod 2 while
+  // the loads of the RGP stages after it are in flight; one barrier a stage
+  // (a slot is refilled two stages later, after every wave has passed the
+  // barrier that follows its last reads of it). The loads of the full stages
+  // are unconditional, past the last one they read it again: a load under a
+  // branch would make the wave wait for every load in flight.
+  static __device__ __forceinline__ void rg_barrier() {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
+    asm volatile("s_barrier" ::: "memory");
+  }
+  template <bool LOADS, bool COMPUTES, typename Slots>
+  __device__ __forceinline__ void rg_rounds(const Slots& slots, int64_t nfull, int64_t nst,
+                                            int64_t nsteps, f32x4_t (&acc)[CHAINS][FM][FN]) const {
+    RStage st[LOADS ? RGP : 1];
+    if (nfull > 0) {
+      if constexpr (LOADS) {
+#pragma unroll
+        for (int u = 0; u < RGP; u++) rg_load(min((int64_t)u, nfull - 1), st[u]);
+      }
+      int64_t s0 = 0;
+      for (; s0 + RGP <= nfull; s0 += RGP) {
+#pragma unroll
+        for (int u = 0; u < RGP; u++) {
+          if constexpr (LOADS) {
+            rg_store(slots(u & 1), st[u]);
+            rg_load(min(s0 + u + RGP, nfull - 1), st[u]);
+          }
+          rg_barrier();
+          if constexpr (COMPUTES) compute_full(slots(u & 1), acc);
+        }
+      }
+#pragma unroll
+      for (int u = 0; u < RGP - 1; u++) {
+        if (s0 + u < nfull) {
+          if constexpr (LOADS) rg_store(slots(u & 1), st[u]);
+          rg_barrier();
+          if constexpr (COMPUTES) compute_full(slots(u & 1), acc);
+        }
+      }
+    }
+    for (int64_t s = nfull; s < nst; s++) {
+      const Slot slot = (s & 1) ? slots(1) : slots(0);
+      if constexpr (LOADS) {
+        rg_load_tail(s, st[0]);
+        rg_store(slot, st[0]);
+      }
+      rg_barrier();
+      if constexpr (COMPUTES) compute(slot, steps_of(nsteps, s), acc);
+    }
+  }
+
   template <typename Slots>
-  __device__ __forceinline__ void main_loop_slow(const Slots& slots, int64_t nst,
-                                                 int64_t nsteps, bool computes,
-                                                 f32x4_t (&acc)[CHAINS][FM][FN]) const {
-    uint4 ra[LA], rb[LB];
-    for (int64_t s = 0; s < nst; s++) {
-      gload_slow(s, ra, rb);
-      Slot slot = (s & 1) ? slots(1) : slots(0);
-      sstore(slot, ra, rb);
-      __syncthreads();
-      if (computes) compute(slot, steps_of(nsteps, s), acc);
-      __syncthreads();
+  __device__ __forceinline__ void main_loop_ragged(const Slots& slots, int64_t nst,
+                                                   int64_t nsteps, bool computes,
+                                                   f32x4_t (&acc)[CHAINS][FM][FN]) {
+    const int64_t kf = kfull();
+    const int64_t nfull = kf > 0 ? kf / EPS : 0;
+    if constexpr (RNT < NT) {
+      if (wave >= CW) {
+        init_ragged();
+        rg_rounds<true, false>(slots, nfull, nst, nsteps, acc);
+      } else if (computes) {
+        rg_rounds<false, true>(slots, nfull, nst, nsteps, acc);
+      } else {
+        rg_rounds<false, false>(slots, nfull, nst, nsteps, acc);
+      }
+    } else {
+      init_ragged();
+      if (computes)
+        rg_rounds<true, true>(slots, nfull, nst, nsteps, acc);
+      else
+        rg_rounds<true, false>(slots, nfull, nst, nsteps, acc);
     }
   }
 };
 
+// RG: the register-staged kernel for operands that are not 16-byte aligned
+// (NS = 2).
 template <typename T, int BM, int BN, int WM, int WN, int NW, int KB, int NS, bool TB, bool PL,
-          bool PP>
+          bool PP, bool RG>
 __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
   using Tile = GemmTile<T, BM, BN, WM, WN, NW, KB, NS, TB, 0, PL, PP>;
   constexpr int FM = Tile::FM, FN = Tile::FN, CHAINS = Tile::CHAINS;
@@ -1342,7 +1485,9 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
       for (int jn = 0; jn < FN; jn++) acc[ch][i][jn] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   t.init_lds_offsets();
-  if (p.vec_a && p.vec_b) {
+  if constexpr (RG) {
+    t.main_loop_ragged(slots, nst, nsteps, computes, acc);
+  } else {
     t.init_buffers();
     if constexpr (PP) {
       t.main_loop_pp(slots, nst, computes, acc);
@@ -1351,20 +1496,14 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
       if (!PL || t.wave >= Tile::CW) t.init_dma();
       t.main_loop_dma(slots, nst, computes, acc);
     }
-  } else if constexpr (!PL && !PP) {
-    // PL and PP footprints take 16-byte aligned operands only: the host
-    // launches another footprint for the others (the slow path's registers
-    // would make the whole kernel spill).
-    t.main_loop_slow(slots, nst, nsteps, computes, acc);
   }
 
-  // Epilogue: one rounding per element. A wave whose sub-tile lies wholly
-  // inside C, with 16-byte aligned output rows, rounds its tile into LDS
-  // (the ring is free once every wave is past the loop and no load is in
-  // flight) and stores it back row by row with 16-byte stores, so each row
-  // of the tile is written as whole cache lines. Otherwise (C's edges,
-  // unaligned rows) each lane stores its own elements. Both store the same
-  // values.
+  // Epilogue: one rounding per element. A wave whose columns lie wholly
+  // inside C rounds its tile into LDS (the ring is free once every wave is
+  // past the loop and no load is in flight) and stores its rows inside C
+  // with 16-byte stores (of any alignment, for a C whose rows have none), so
+  // each row of the tile is written as whole cache lines. Otherwise (C's last
+  // columns) each lane stores its own elements. Both store the same values.
   constexpr int SWB = Tile::WTM * Tile::WTN * (int)sizeof(T);  // staged bytes per wave
   constexpr int WPA = AC * 16 / SWB;                            // waves per A array
   constexpr int WPB = BC * 16 / SWB;                            // waves per B array
@@ -1380,8 +1519,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
   const T* __restrict__ bias = static_cast<const T*>(p.bias);
   const float alpha = p.alpha, beta = p.beta;
   if constexpr (STAGED) {
-    const bool whole = wrow + Tile::WTM <= M && wcol + Tile::WTN <= N &&
-                       N % Tile::EPC == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0;
+    const bool whole = wcol + Tile::WTN <= N;
     if (whole) {
       T* stage;
       if constexpr (STAGED_A) {
@@ -1411,9 +1549,9 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
 #pragma unroll
       for (int r0 = 0; r0 < Tile::WTM; r0 += RPI) {
         const int r = r0 + t.lane / CPRW, c = t.lane % CPRW;
-        if (Tile::WTM % RPI == 0 || r < Tile::WTM) {
+        if ((Tile::WTM % RPI == 0 || r < Tile::WTM) && wrow + r < M) {
           const uint4 v = reinterpret_cast<const uint4*>(stage)[r * CPRW + c];
-          *reinterpret_cast<uint4*>(out + (wrow + r) * N + wcol + c * Tile::EPC) = v;
+          __builtin_memcpy(out + (wrow + r) * N + wcol + c * Tile::EPC, &v, 16);
         }
       }
       return;
@@ -1539,13 +1677,22 @@ using KernelFn = void (*)(GemmArgs);
 
 namespace bi_gemm_dev {
 
-// Kernel for geometry g in the translation unit of element type T.
+// Kernel for geometry g in the translation unit of element type T; ragged:
+// its register-staged form for operands that are not 16-byte aligned (the
+// footprints with loading waves or more than 8 waves have none: the staged
+// loads' registers would make them spill).
 template <typename T>
-KernelFn kernel_for(int g, bool trans_b) {
+KernelFn kernel_for(int g, bool trans_b, bool ragged) {
 // fp32 carries two accumulator chains per element: with more than 8 waves
 // (at most 168 registers each) the 64 x 64 wave tiles do not fit.
 #define BI_GEO_CASE(id, bm, bn, wm, wn, nw, kb, ns, pl, pp)                             \
   case id:                                                                             \
+    if (ragged) {                                                                      \
+      if constexpr (!pl && !pp)                                                        \
+        return trans_b ? gemm_kernel<T, bm, bn, wm, wn, nw, kb, 2, true, 0, 0, true>   \
+                       : gemm_kernel<T, bm, bn, wm, wn, nw, kb, 2, false, 0, 0, true>; \
+      return nullptr;                                                                  \
+    }                                                                                  \
     if constexpr (pp == 2) {                                                           \
       if constexpr (sizeof(T) == 2)                                                    \
         return trans_b ? gemm_w4_kernel<T, true> : gemm_w4_kernel<T, false>;           \
@@ -1554,8 +1701,10 @@ KernelFn kernel_for(int g, bool trans_b) {
     } else if constexpr (sizeof(T) == 4 && (nw > 8 || pp)) {                           \
       return nullptr;                                                                  \
     } else {                                                                           \
-      return trans_b ? gemm_kernel<T, bm, bn, wm, wn, nw, kb, ns, true, pl, pp != 0>   \
-                     : gemm_kernel<T, bm, bn, wm, wn, nw, kb, ns, false, pl, pp != 0>; \
+      return trans_b ? gemm_kernel<T, bm, bn, wm, wn, nw, kb, ns, true, pl, pp != 0,   \
+                                   false>                                              \
+                     : gemm_kernel<T, bm, bn, wm, wn, nw, kb, ns, false, pl, pp != 0,  \
+                                   false>;                                             \
     }
   switch (g) { BI_GEOMETRIES(BI_GEO_CASE) }
 #undef BI_GEO_CASE
@@ -1626,9 +1775,9 @@ KernelFn qdecode_kernel_for(int group, int rows, int bits) {
 }  // namespace bi_gemm_dev
 
 // Per-type kernel tables, defined in bi_gemm_{f32,f16,bf16}.hip.
-bi_gemm_dev::KernelFn bi_gemm_kernel_f32(int g, bool trans_b);
-bi_gemm_dev::KernelFn bi_gemm_kernel_f16(int g, bool trans_b);
-bi_gemm_dev::KernelFn bi_gemm_kernel_bf16(int g, bool trans_b);
+bi_gemm_dev::KernelFn bi_gemm_kernel_f32(int g, bool trans_b, bool ragged);
+bi_gemm_dev::KernelFn bi_gemm_kernel_f16(int g, bool trans_b, bool ragged);
+bi_gemm_dev::KernelFn bi_gemm_kernel_bf16(int g, bool trans_b, bool ragged);
 bi_gemm_dev::KernelFn bi_qgemm_kernel_f16(int g, int bits, int group);
 bi_gemm_dev::KernelFn bi_qgemm_kernel_bf16(int g, int bits, int group);
 bi_gemm_dev::KernelFn bi_qdecode_kernel_f16(int group, int rows, int bits);

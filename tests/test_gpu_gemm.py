@@ -199,6 +199,50 @@ def test_unaligned_operands_leave_the_aligned_only_footprint(cuda):
                     "%s K=%d geometry %s" % (dname, K, geos[gi]))
 
 
+@pytest.mark.parametrize("trans_b", [False, True])
+@pytest.mark.parametrize("M,K,N", [(1, 1, 1), (3, 7, 5), (2, 3, 2), (17, 9, 17), (33, 129, 65),
+                                   (65, 255, 33), (70, 257, 130), (130, 519, 129), (1, 1001, 40),
+                                   (301, 1001, 303), (16, 512, 3), (16, 1024, 130)])
+def test_ragged_operands(cuda, trans_b, M, K, N):
+    """Operands whose rows are not 16-byte aligned take the register-staged
+    kernels: every footprint that has one gives the bits of the same operands
+    padded with zeros to aligned rows. NaNs in the last row of A and the last
+    column of B, which the tails of the rows before them touch, and around
+    both buffers reach no other output."""
+    geos = _gemm.geometries()
+    for dname, dtype in DTYPES:
+        def odd(shape, seed, std=1.0):
+            buf = torch.full((shape[0] * shape[1] + 65,), float("nan"), dtype=dtype, device=cuda)
+            t = buf[1:1 + shape[0] * shape[1]].view(shape)
+            t.copy_(rn(shape, dtype, seed, std=std, device=cuda))
+            return t
+
+        a = odd((M, K), 51)
+        b = odd((N, K) if trans_b else (K, N), 52, K ** -0.5)
+        c = rn((N,), dtype, 53, device=cuda)
+        if M > 1:
+            a[-1] = float("nan")
+        if N > 1:
+            (b[-1] if trans_b else b[:, -1]).fill_(float("nan"))
+        Kp, Np = -(-K // 8) * 8, -(-N // 8) * 8
+        ap = torch.nn.functional.pad(a, (0, Kp - K))
+        bp = torch.nn.functional.pad(b, (0, Kp - K, 0, Np - N) if trans_b else (0, Np - N, 0, Kp - K))
+        cp = torch.nn.functional.pad(c, (0, Np - N))
+        want = _gemm._gemm(ap, bp, cp, trans_b, 1.5, -0.5)[:, :N]
+        ran = 0
+        for gi in [None] + list(range(len(geos))):
+            try:
+                got = _gemm._gemm(a, b, c, trans_b, 1.5, -0.5, geometry=gi)
+            except NotImplementedError:
+                continue  # footprints that take aligned operands only
+            ran += 1
+            same = (got == want) | (got.isnan() & want.isnan())
+            assert bool(same.all()), "%s geometry %s: %d differ" % (
+                dname, "picked" if gi is None else geos[gi], int((~same).sum()))
+            assert not bool(got[:max(1, M - 1), :max(1, N - 1)].isnan().any())
+        assert ran == 6
+
+
 def test_kn_and_nk_layouts_agree(cuda):
     """matmul on a (K, N) weight and linear on the same weight stored (N, K)
     feed the MFMAs identically, so they give the same bits; a transposed view
