@@ -119,6 +119,18 @@ int bi_sdpa_with_shape(const void* q, const void* k, const void* v,
                        float scale, int mask_mode, int64_t causal_offset,
                        int dtype, int shape, void* hip_stream);
 
+/* bi_sdpa_ws with one segment of the keys per workgroup, in launch shape
+ * `shape` (BI_F16 / BI_BF16; any but "shared"), whatever the size. */
+int bi_sdpa_split_with_shape(const void* q, const void* k, const void* v,
+                             const void* mask, const int64_t* mask_strides,
+                             const void* sinks, void* out,
+                             int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N,
+                             int64_t D, int64_t V,
+                             const int64_t* qkv_strides,
+                             float scale, int mask_mode, int64_t causal_offset,
+                             int dtype, int shape, void* workspace, int64_t workspace_bytes,
+                             void* hip_stream);
+
 /* Wavefront width the kernels were compiled for (64 on gfx950); the fixed
  * reduction shapes assume it. Reads a device-side constant: needs a GPU. */
 int bi_device_wavefront_size(int* out);

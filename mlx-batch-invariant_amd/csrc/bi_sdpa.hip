@@ -32,6 +32,7 @@
 //     out = L == 0 ? o : o / L (reference :124-141), one rounding to T.
 #include <hip/hip_runtime.h>
 #include <float.h>
+#include <math.h>
 #include <atomic>
 #include <stdint.h>
 
@@ -39,6 +40,7 @@
 
 #include "bi_internal.h"
 #include "bi_sdpa_args.h"
+#include "bi_sdpa_fold.h"
 
 namespace {
 
@@ -46,7 +48,6 @@ constexpr int kThreads = 256;
 constexpr int64_t kMaskSlack = 64;  // keys a block may read past N
 constexpr int kPartials = 32;
 constexpr int kGroupLanes = 8;
-constexpr float kLog2e = 1.4426950408889634f;
 
 template <typename T> __device__ inline float to_f32(T x) { return (float)x; }
 // A mask element held as its zero-extended bits (16-bit types) or as itself
@@ -368,9 +369,47 @@ SdpaKernelFn f32_kernel(int64_t D, int64_t V, int shape) {
 
 // ---------------------------------------------------------------- MFMA shapes
 
-SdpaKernelFn mfma_kernel(int64_t D, int64_t V, int dtype, bool mask, int shape) {
+// Folds the segments' partial results (SdpaArgs::part) in ascending order and
+// writes the output; one thread per column and 4 dims. Bound by the launch and
+// one round of loads, eight segments at a time (about 2.5 us in all).
+template <typename T>
+__global__ void __launch_bounds__(256) sdpa_fold_kernel(SdpaArgs p, int V) {
+  const int quads = V / 4;
+  const int64_t ncol = p.B * p.H * p.qL;
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t col = i / quads;
+  if (col >= ncol) return;
+  const int d = (int)(i % quads) * 4;
+  const float* __restrict__ po = p.part + col * p.nseg * V + d;
+  const float2* __restrict__ pm =
+      reinterpret_cast<const float2*>(p.part + ncol * p.nseg * V) + col * p.nseg;
+  // (The fold of the first segment into this state leaves it as it is.)
+  float R = -FLT_MAX, S = 0.f;
+  f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  constexpr int A = 8;
+  for (int s0 = 0; s0 < p.nseg; s0 += A) {
+    f32x4_t O[A];
+    float2 st[A];
+#pragma unroll
+    for (int u = 0; u < A; u++) {
+      const int s = s0 + u < p.nseg ? s0 + u : p.nseg - 1;
+      O[u] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)s * V);
+      st[u] = pm[s];
+    }
+#pragma unroll
+    for (int u = 0; u < A; u++)
+      if (s0 + u < p.nseg) fold_out(Q, O[u], fold_stats(R, S, st[u].x, st[u].y));
+  }
+  unsigned short ob[4];
+#pragma unroll
+  for (int e = 0; e < 4; e++) ob[e] = __builtin_bit_cast(unsigned short, (T)(S == 0.f ? Q[e] : Q[e] / S));
+  *reinterpret_cast<uint2*>(static_cast<T*>(p.out) + col * V + d) =
+      make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
+}
+
+SdpaKernelFn mfma_kernel(int64_t D, int64_t V, int dtype, bool mask, int shape, int seg) {
 #define BI_MFMA_CASE(d, v) \
-  if (D == d && V == v) return sdpa_mfma_kernel_d##d##_v##v(dtype, mask, shape);
+  if (D == d && V == v) return sdpa_mfma_kernel_d##d##_v##v(dtype, mask, shape, seg);
   BI_SDPA_DIM_PAIRS(BI_MFMA_CASE)
 #undef BI_MFMA_CASE
   return nullptr;
@@ -445,20 +484,86 @@ bool shape_geometry(int64_t D, int64_t V, int dtype, int shape, int* columns, in
     *splits = 1;
     return true;
   }
-  if (shape < 0 || shape >= SDPA_NUM_SHAPES || !mfma_kernel(D, V, dtype, false, shape))
+  if (shape < 0 || shape >= SDPA_NUM_SHAPES || !mfma_kernel(D, V, dtype, false, shape, SEG_ONE))
     return false;
   *columns = sdpa_shape_columns(D, V, shape);
   *splits = sdpa_shape_splits(V, shape);
   return true;
 }
 
+int64_t segments(int64_t N) { return N > 0 ? (N + kSegKeys - 1) / kSegKeys : 1; }
+
+// Bytes of partial results (SdpaArgs::part) of a launch over segments.
+int64_t split_bytes(int64_t B, int64_t H, int64_t qL, int64_t N, int64_t V) {
+  return B * H * qL * segments(N) * (V + 2) * (int64_t)sizeof(float);
+}
+
+// Estimated microseconds of a matrix-core launch whose workgroups each walk
+// `keys` of a segment's (or, nseg 1, of the whole context's) keys: the longest
+// of a chain's own time for its blocks, the key and value bytes that leave
+// HBM once per stream, and those that reach the workgroups through the L2s,
+// plus 4.5 for the launch's fixed parts. Fitted to a grid of B = 1..64, N =
+// 2100..8192, 1..32 query rows, D = 64, 128, 256, with and without an array
+// mask; a loader-wave workgroup fills a CU, so a few of them past a multiple
+// of the CUs cost a round.
+float estimate(int64_t D, int64_t V, int64_t tiles, int64_t streams, int shape, bool array_mask,
+               int64_t nseg, float keys, float walk, int cus) {
+  const bool loaders = sdpa_loaders(D, V, shape, array_mask);
+  const bool rows = shape == SDPA_ROWS && sdpa_rows_tiles(D, V) == 2;
+  const int ws = sdpa_shape_splits(V, shape);
+  const float dv = (float)(D + V), inv = 1.f / (float)ws;
+  const float chain = loaders ? 10.6f + 0.4f * inv                    // per 2048 keys
+                      : rows  ? 0.09f * dv
+                              : 6.f + (0.045f + 0.012f * inv) * dv;
+  float wgs = (float)((rows ? (tiles + streams) / 2 : tiles) * ws * nseg) / (float)cus;
+  if (loaders && wgs > 1.f) wgs = ceilf(wgs);
+  float hbm = 0.184f * dv * (float)(streams * nseg) / (float)cus;
+  if (ws == 1 && wgs < 1.f) hbm *= 1.15f;
+  if (nseg > 1) hbm *= 1.08f;
+  const float l2 = (rows ? (array_mask ? 0.15f : 0.105f) * dv
+                         : (nseg > 1 ? 0.132f : ws == 1 ? 0.09f : ws == 2 ? 0.075f : 0.098f) *
+                               ((float)D + (float)V * inv)) * wgs;
+  const float a = chain * walk / 2048.f, b = (hbm > l2 ? hbm : l2) * keys / 2048.f;
+  return 4.5f + (a > b ? a : b);
+}
+
+// The launch shape of a launch over segments, or -1 where one workgroup
+// should walk every segment: a grid that leaves compute units idle, or whose
+// dim-split workgroups each stream every key (B = 1, N = 8192, D = 128: 31 us
+// by 64 workgroups of 8-way split dims, 16 us over 4 segments; B = 4: 55 and
+// 30 us; B = 16: 93 and 101 us). Short second segments are not worth the fold's
+// launch, about 2.5 us (N = 2100: 13 and 15 us; N = 3000: the same).
+int pick_split(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
+               int dtype, int mask_mode, int cus) {
+  if (dtype == BI_F32 || N <= kSegKeys + kSegKeys / 2) return -1;
+  const bool am = mask_mode == BI_MASK_ARRAY;
+  const int64_t streams = B * Hkv, ncol = (H / Hkv) * qL;
+  const int64_t tiles = streams * ((ncol + 15) / 16), ns = segments(N);
+  const int walk = pick_shape(B, H, Hkv, qL, D, V, dtype, mask_mode, cus);
+  if (walk == SDPA_SHARED) return -1;
+  float best = estimate(D, V, tiles, streams, walk, am, 1, (float)N, (float)N, cus);
+  int shape = -1;
+  for (int s = SDPA_ROWS; s <= SDPA_SPLIT8; s++) {
+    if (s == SDPA_ROWS && (ncol <= 16 || sdpa_rows_tiles(D, V) != 2)) continue;
+    const float t = 1.05f * (2.5f + estimate(D, V, tiles, streams, s, am, ns, (float)N / (float)ns,
+                                             (float)kSegKeys, cus));
+    if (t < best) {
+      best = t;
+      shape = s;
+    }
+  }
+  return shape;
+}
+
 // Validates, packs the arguments and launches shape `shape` (-1: the shape
-// bi_sdpa picks).
+// bi_sdpa picks). `ws`, `ws_bytes`: memory for partial results, which lets a
+// launch take one segment of the keys per workgroup: with `split` it must
+// (shape says which), else it does where pick_split says so.
 int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
              const int64_t* mask_strides, const void* sinks, void* out, int64_t B, int64_t H,
              int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
              const int64_t* qkv_strides, float scale, int mask_mode, int64_t causal_offset,
-             int dtype, int shape, void* hip_stream) {
+             int dtype, int shape, bool split, void* ws, int64_t ws_bytes, void* hip_stream) {
   const int esz = bi::elem_size(dtype);
   if (!esz) return bi::fail(BI_EINVAL, "bi_sdpa: unknown dtype %d", dtype);
   if (B < 0 || H <= 0 || Hkv <= 0 || qL < 0 || N < 0 || D <= 0 || V <= 0)
@@ -531,6 +636,22 @@ int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
         ((H - 1) * p.ms[1] + (qL - 1) * p.ms[2] + N + kMaskSlack) * esz > INT32_MAX)
       return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: the mask of one batch entry is too large");
   }
+  p.part = nullptr;
+  p.nseg = 1;
+  if (split && (dtype == BI_F32 || shape == SDPA_SHARED))
+    return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: launch shape %d is not built over segments", shape);
+  const int64_t need = split_bytes(B, H, qL, N, V);
+  if (!split && shape < 0 && ws && ws_bytes >= need) {
+    shape = pick_split(B, H, Hkv, qL, N, D, V, dtype, mask_mode, device_cus());
+    split = shape >= 0;
+  }
+  if (split) {
+    if (!ws || (uintptr_t)ws % 16 || ws_bytes < need)
+      return bi::fail(BI_EINVAL, "bi_sdpa: the workspace needs %lld bytes, 16-byte aligned",
+                      (long long)need);
+    p.part = static_cast<float*>(ws);
+    p.nseg = (int)segments(N);
+  }
   if (shape < 0) shape = pick_shape(B, H, Hkv, qL, D, V, dtype, mask_mode, device_cus());
   int columns = 0, splits = 0;
   if (!shape_geometry(D, V, dtype, shape, &columns, &splits))
@@ -547,9 +668,10 @@ int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
     fn = f32_kernel(D, V, shape);
     blocks = rows / columns;
   } else {
-    fn = mfma_kernel(D, V, dtype, mask_mode == BI_MASK_ARRAY, shape);
+    fn = mfma_kernel(D, V, dtype, mask_mode == BI_MASK_ARRAY, shape,
+                     split ? SEG_SPLIT : N > kSegKeys ? SEG_WALK : SEG_ONE);
     const int64_t ncol = (H / Hkv) * qL;
-    blocks = B * Hkv * ((ncol + columns - 1) / columns) * splits;
+    blocks = B * Hkv * ((ncol + columns - 1) / columns) * splits * p.nseg;
   }
   if (blocks > INT32_MAX) return bi::fail(BI_EINVAL, "bi_sdpa: grid too large");
   if (!fn)
@@ -558,8 +680,19 @@ int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
       dtype == BI_F32 ? kThreads : sdpa_shape_threads(D, V, shape, mask_mode == BI_MASK_ARRAY);
   hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(threads), 0,
                      static_cast<hipStream_t>(hip_stream), p);
-  const hipError_t e = hipGetLastError();
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return bi::launch_error(e, "bi_sdpa launch");
+  if (p.part) {
+    const int64_t fold_blocks = (rows * (V / 4) + 255) / 256;  // rows <= 2^31, V <= 512
+    if (dtype == BI_BF16)
+      hipLaunchKernelGGL(sdpa_fold_kernel<__bf16>, dim3((unsigned)fold_blocks), dim3(256), 0,
+                         static_cast<hipStream_t>(hip_stream), p, (int)V);
+    else
+      hipLaunchKernelGGL(sdpa_fold_kernel<_Float16>, dim3((unsigned)fold_blocks), dim3(256), 0,
+                         static_cast<hipStream_t>(hip_stream), p, (int)V);
+    e = hipGetLastError();
+    if (e != hipSuccess) return bi::launch_error(e, "bi_sdpa fold launch");
+  }
   return BI_OK;
 }
 
@@ -571,7 +704,41 @@ extern "C" int bi_sdpa(const void* q, const void* k, const void* v, const void* 
                        const int64_t* qkv_strides, float scale, int mask_mode,
                        int64_t causal_offset, int dtype, void* hip_stream) {
   return sdpa_run(q, k, v, mask, mask_strides, sinks, out, B, H, Hkv, qL, N, D, V, qkv_strides,
-                  scale, mask_mode, causal_offset, dtype, -1, hip_stream);
+                  scale, mask_mode, causal_offset, dtype, -1, false, nullptr, 0, hip_stream);
+}
+
+extern "C" int64_t bi_sdpa_workspace(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N,
+                                     int64_t D, int64_t V, int dtype, int mask_mode) {
+  if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || qL <= 0 || !dims_built(D, V)) return 0;
+  if (N > INT32_MAX - 1024 || B * H * qL > INT32_MAX) return 0;
+  return pick_split(B, H, Hkv, qL, N, D, V, dtype, mask_mode, device_cus()) < 0
+             ? 0
+             : split_bytes(B, H, qL, N, V);
+}
+
+extern "C" int bi_sdpa_ws(const void* q, const void* k, const void* v, const void* mask,
+                          const int64_t* mask_strides, const void* sinks, void* out, int64_t B,
+                          int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
+                          const int64_t* qkv_strides, float scale, int mask_mode,
+                          int64_t causal_offset, int dtype, void* workspace,
+                          int64_t workspace_bytes, void* hip_stream) {
+  return sdpa_run(q, k, v, mask, mask_strides, sinks, out, B, H, Hkv, qL, N, D, V, qkv_strides,
+                  scale, mask_mode, causal_offset, dtype, -1, false, workspace, workspace_bytes,
+                  hip_stream);
+}
+
+extern "C" int bi_sdpa_split_with_shape(const void* q, const void* k, const void* v,
+                                        const void* mask, const int64_t* mask_strides,
+                                        const void* sinks, void* out, int64_t B, int64_t H,
+                                        int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
+                                        const int64_t* qkv_strides, float scale, int mask_mode,
+                                        int64_t causal_offset, int dtype, int shape,
+                                        void* workspace, int64_t workspace_bytes,
+                                        void* hip_stream) {
+  if (shape < 0) return bi::fail(BI_EINVAL, "bi_sdpa_split_with_shape: shape %d", shape);
+  return sdpa_run(q, k, v, mask, mask_strides, sinks, out, B, H, Hkv, qL, N, D, V, qkv_strides,
+                  scale, mask_mode, causal_offset, dtype, shape, true, workspace, workspace_bytes,
+                  hip_stream);
 }
 
 extern "C" int bi_sdpa_with_shape(const void* q, const void* k, const void* v, const void* mask,
@@ -582,7 +749,7 @@ extern "C" int bi_sdpa_with_shape(const void* q, const void* k, const void* v, c
                                   void* hip_stream) {
   if (shape < 0) return bi::fail(BI_EINVAL, "bi_sdpa_with_shape: shape %d", shape);
   return sdpa_run(q, k, v, mask, mask_strides, sinks, out, B, H, Hkv, qL, N, D, V, qkv_strides,
-                  scale, mask_mode, causal_offset, dtype, shape, hip_stream);
+                  scale, mask_mode, causal_offset, dtype, shape, false, nullptr, 0, hip_stream);
 }
 
 extern "C" int bi_sdpa_pick_shape(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t D,

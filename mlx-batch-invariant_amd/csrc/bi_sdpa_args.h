@@ -24,7 +24,20 @@ struct SdpaArgs {
   uint32_t qsign;
   int mask_mode;
   int64_t causal_offset;
+  // SEG_SPLIT kernels: each workgroup takes one segment of kSegKeys keys (nseg
+  // of them) and leaves its columns' partial results here for
+  // sdpa_fold_kernel: O[column][segment][V], then (M, L)[column][segment],
+  // column = (b * H + head) * qL + row.
+  float* part;
+  int nseg;
 };
+
+// How a matrix-core kernel treats the segments of the keys: there is one
+// (N <= kSegKeys); its workgroups walk them all and fold them; or each
+// workgroup takes one and sdpa_fold_kernel folds them. The same arithmetic.
+enum SdpaSeg { SEG_ONE = 0, SEG_WALK = 1, SEG_SPLIT = 2 };
+// Keys per segment of the matrix-core kernels' fixed arithmetic.
+constexpr int kSegKeys = 2048;
 
 typedef void (*SdpaKernelFn)(SdpaArgs);
 
@@ -91,9 +104,9 @@ constexpr int sdpa_shape_threads(int64_t D, int64_t V, int shape, bool array_mas
                                                      : 256;
 }
 
-// The MFMA kernel of one head-dim pair for (dtype, array mask or not, shape);
-// nullptr for an element type it is not built for (bi_sdpa_mfma_d*.hip).
+// The MFMA kernel of one head-dim pair for (dtype, array mask or not, shape,
+// SdpaSeg); nullptr where there is none (bi_sdpa_mfma_d*.hip).
 #define BI_SDPA_MFMA_DECLARE(D, V) \
-  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape);
+  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int seg);
 BI_SDPA_DIM_PAIRS(BI_SDPA_MFMA_DECLARE)
 #undef BI_SDPA_MFMA_DECLARE

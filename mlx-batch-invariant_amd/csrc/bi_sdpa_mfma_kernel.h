@@ -6,16 +6,18 @@
 // with matrix cores: one workgroup owns the whole key reduction for each of
 // its query columns -- a column is one (query head, query row) pair; the
 // columns of a workgroup share a batch index and a kv head, so they read the
-// same keys and values -- with no split-KV, no second pass and no switch on
-// query length or context length. The workgroup's 4 waves walk the keys in a
+// same keys and values -- or, where the grid would leave the chip idle, one
+// segment of it, at fixed keys, its partial results folded by a second kernel
+// in the order the first would have. The workgroup's 4 waves walk the keys in a
 // fixed stride order (the reference's fixed per-simdgroup strides, :89) and
 // their partial results are merged in a fixed order through LDS (:124-141).
 // D is the query/key head dim and V the value head dim (both multiples of 32,
 // reference :33-34, :224-227).
 //
 // Fixed per-column arithmetic (the invariance contract):
-//   * Keys are taken in blocks of 32 (block b = keys 32b .. 32b + 31). Block b
-//     belongs to chain b mod 4; each chain walks its blocks in ascending order.
+//   * Keys are taken in segments of 2048 (fixed positions) and blocks of 32
+//     (block b = keys 32b .. 32b + 31). Block b belongs to chain b mod 4 of its
+//     segment; each chain walks its blocks in ascending order.
 //   * Score: raw_i = q . k_i as a chain of v_mfma_f32_16x16x32_{bf16,f16}
 //     over the head dim in ascending 32-element chunks from +0.0 (exact
 //     products, fp32 sums). With a = |scale| * log2 e (a negative scale
@@ -23,7 +25,7 @@
 //     score is s_i = raw_i * a, plus mask_i * log2 e for an additive mask.
 //   * Key i is used iff i < N, i <= row + causal_offset (causal) and
 //     mask_i > -3e38 (array mask) (reference :92-96).
-//   * Each chain runs an online softmax in base 2 over its blocks: with M the
+//   * Each chain of a segment runs an online softmax in base 2 over its blocks: with M the
 //     largest used s_i of the block (without a mask taken as max_i(raw_i) * a,
 //     the same value since rounding is monotonic; none used: the block leaves
 //     the chain unchanged), m' = M > m + 8 ? M : m (a lazily moved base),
@@ -37,14 +39,21 @@
 //     keys 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3. m starts at the lowest
 //     finite float and l at 0 (reference :76-79). A mask of zeros gives the
 //     bits of no mask.
-//   * Merge: a sink (reference :80-86, an extra denominator term exp(sink))
-//     enters here as one more partial with m = sink * log2 e, l = 1, o = 0,
-//     ahead of the chains: M = max of the sink's and the chains' m;
-//     L = exp2(sink2 - M) (0 without a sink), O = +0.0; then for
-//     c = 0, 1, 2, 3 in order, e_c = exp2(m_c - M), L = fma(l_c, e_c, L) and
-//     O = fma(o_c, e_c, O); out = L == 0 ? O : O / L, one rounding to T.
+//   * A segment's chains merge in order: M = max of the chains' m; L = 0,
+//     O = +0.0; then for c = 0, 1, 2, 3, e_c = exp2(m_c - M),
+//     L = fma(l_c, e_c, L) and O = fma(o_c, e_c, O). A sink (reference :80-86,
+//     an extra denominator term exp(sink)) enters the first segment's merge as
+//     one more partial with m = sink * log2 e, l = 1, o = 0, ahead of the
+//     chains: M is the max with it too, and L starts at exp2(sink2 - M).
 //     (Seeding a chain's base with the sink, as the reference seeds its
 //     simdgroup 0, would put a large sink's p below f16's range.)
+//   * The segments fold in ascending order: the first segment's (M, L, O) is
+//     the running (R, S, Q); then R' = max(R, M), e = exp2(R - R'),
+//     f = exp2(M - R'), S = fma(L, f, S * e), Q = fma(O, f, fma(Q, e, 0))
+//     (never -0.0, so a segment without a usable key changes no bit).
+//     out = S == 0 ? Q : Q / S, one rounding to T.
+//     Segments lie at fixed keys, so whether one workgroup walks them all or
+//     each has its own workgroup changes nothing a column computes.
 // Every column, whatever workgroup or lane it lands in, however many rows or
 // heads share its keys and whatever the launch shape (columns per workgroup,
 // prefetch depths), runs exactly this sequence: an output row has the same
@@ -60,6 +69,7 @@
 
 #include "bi_internal.h"
 #include "bi_sdpa_args.h"
+#include "bi_sdpa_fold.h"
 
 namespace {
 
@@ -67,7 +77,6 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -85,7 +94,8 @@ __device__ __forceinline__ void st16(uint4* p, uint4 v) {
 constexpr int kWaves = 4;  // = chains
 constexpr int kThreads = 64 * kWaves;
 constexpr int kBlk = 32;   // keys per block
-constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kSegBlk = kSegKeys / kBlk;      // blocks per segment
+constexpr int kSegIt = kSegBlk / kWaves;      // of them in one chain
 
 // s_waitcnt immediates (gfx9 encoding: vmcnt [3:0] + [15:14], expcnt [6:4],
 // lgkmcnt [11:8]).
@@ -145,6 +155,13 @@ __device__ __forceinline__ u32x4_t ds_read_b128_at(uint32_t lds_addr, int off) {
   u32x4_t v;
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "i"(off) : "memory");
   return v;
+}
+
+// A 16-byte LDS write of matrix-product results as an asm statement. The
+// compiler does not count the wait states between an MFMA and an asm
+// statement that reads its result; 24 cover every MFMA used here.
+__device__ __forceinline__ void ds_write_acc(uint32_t lds_addr, f32x4_t v) {
+  asm volatile("s_nop 15\n\ts_nop 7\n\tds_write_b128 %0, %1" ::"v"(lds_addr), "v"(v) : "memory");
 }
 
 template <typename T> __device__ inline unsigned short tbits(T x) {
@@ -295,7 +312,7 @@ struct Chain {
   const T* mb;
   int64_t ks2, vs2, N, mext;
   int nit;
-  int wave;
+  int wave;  // the chain's first block (block i of the chain: wave + 4i)
   // Lane byte offsets: key row 16kt + r16 at dims 8g ..; value chunk j;
   // mask keys 4g .. of the lane's row in each column tile. The other key and
   // mask loads add constants (immediate offsets, which the range check
@@ -407,8 +424,8 @@ struct Chain {
 // LW: 0, or kWaves loader waves (keys in LDS only). A loader wave issues the
 // loads of one chain's blocks, so the chain wave's instruction stream holds
 // no load issue (which stalls while the memory pipeline is busy).
-template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW>
-__global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs p) {
+template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
+__device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
   static_assert(LW == 0 || (LW == kWaves && KL && PK == 0 && SV >= 3), "loader waves: one per chain");
   using C = Chain<T, D, V, CT, PK, SV, WS, MK, KL>;
   constexpr int NQ = C::NQ, NB = C::NB, VCH = C::VCH;
@@ -434,9 +451,15 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
   const int64_t G = p.H / p.Hkv;
   const int64_t ncol = G * p.qL;
   const int64_t ncb = (ncol + COLS - 1) / COLS;
-  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * ncb * WS));
+  const int nsplit = SEG == SEG_SPLIT ? p.nseg : 1;
+  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * ncb * WS * nsplit));
   const int ws = (int)(t % WS);
   t /= WS;
+  int seg = 0;  // SEG_SPLIT: this workgroup's
+  if constexpr (SEG == SEG_SPLIT) {
+    seg = (int)(t % nsplit);
+    t /= nsplit;
+  }
   // Causal: the last column blocks see the most keys; they start first.
   const int64_t cb = p.mask_mode == BI_MASK_CAUSAL ? ncb - 1 - t % ncb : t % ncb;
   t /= ncb;
@@ -455,7 +478,12 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
   const int64_t kmax = kend_of(last_cc / G);  // keys some column of the workgroup sees
   // Block counts and indices fit in 32 bits (the host bounds N below
   // 2^31 - 1024), which keeps the loop's compares on the scalar unit.
-  const int nblk = (int)((kmax + kBlk - 1) / kBlk);
+  // This workgroup's blocks: blk0 .. blk0 + nblk - 1, in nsg segments.
+  const int blk0 = seg * kSegBlk;
+  int nblk = (int)((kmax + kBlk - 1) / kBlk);
+  if constexpr (SEG == SEG_SPLIT)
+    nblk = nblk <= blk0 ? 0 : nblk - blk0 < kSegBlk ? nblk - blk0 : kSegBlk;
+  const int nsg = SEG == SEG_WALK ? (nblk + kSegBlk - 1) / kSegBlk : 1;
   const int nfull = (int)(kend_of(c0 / G) / kBlk);  // blocks every column of the workgroup sees
 
   // This lane's column in each tile; its query as the B operand of the score
@@ -488,11 +516,11 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
   // Key and value rows of the stream; per-block buffer resources start at the
   // block's first row, so the lane offsets below are the same for every block
   // (and below 2^31: the host bounds 32 * stride).
-  // This chain's blocks are wave + 4i, i < nit.
+  // This chain's blocks are blk0 + wave + 4i, i < nit.
   const int nit = nblk > wave ? (nblk - wave + kWaves - 1) / kWaves : 0;
   const int wslot = wave * C::VSLOT;  // this wave's slot within each array
   C ld;
-  ld.init(p, b, kvh, ws, wave, nit, lane, mrow, kmax);
+  ld.init(p, b, kvh, ws, blk0 + wave, nit, lane, mrow, kmax);
   // With loader waves every wave runs the same number of steps (chain 0 has
   // the most blocks), one barrier each. PIPE (four slots or more): at step j
   // a chain wave reads and scores the keys of block j while it finishes block
@@ -503,6 +531,11 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
   constexpr bool PIPE = LW != 0 && SV >= 4;
   constexpr int AHEAD = PIPE ? SV - 2 : SV - 1;
   const int steps = PIPE ? nit0 + 1 : nit0;
+  // Whether each chain's first n blocks end a segment that another follows:
+  // the chains then merge before the next (one more barrier with loader waves).
+  auto ends_segment = [&](int n) __attribute__((always_inline)) -> bool {
+    return SEG == SEG_WALK && n % kSegIt == 0 && n > 0 && n < nsg * kSegIt;
+  };
   if constexpr (LW != 0) {
     if (loader) {
       // Block j lands in slot j % SV. Before barrier j this wave waits for
@@ -520,6 +553,7 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
           __builtin_amdgcn_s_waitcnt(wait_vm((AHEAD - 1) * (C::DK + C::DV)));
           asm volatile("s_barrier" ::: "memory");
           ld.vload(j0 + u + AHEAD, arr((u + AHEAD) % SV) + wslot);
+          if (ends_segment(PIPE ? j0 + u : j0 + u + 1)) asm volatile("s_barrier" ::: "memory");
         }
       }
       // The merge below reuses the slots: no load may still be landing
@@ -762,6 +796,148 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
     update(std::false_type{}, sc, mk, slot, blk, va);
   };
 
+  // The running state over the segments so far: (R, S) of each column, and Q
+  // of the dim blocks wave, wave + 4, ... this wave writes out. With two
+  // column tiles, Q lives in LDS between its uses, once in 2048 keys, where
+  // two workgroups' LDS allows, and else all of it in scratch memory
+  // (volatile): two such workgroups share a CU, and their chains' state fills
+  // the 256 registers that leaves a wave.
+  constexpr int KB = (NB + kWaves - 1) / kWaves;
+  constexpr bool QLDS = CT == 2 && SEG == SEG_WALK &&
+                        SV * C::ARR_U4 * 16 + CT * kWaves * KB * 1024 + 1024 <= 80 * 1024;
+  constexpr bool RMEM = CT == 2 && SEG == SEG_WALK && !QLDS;
+  struct Run {
+    float R, S;
+    f32x4_t Q[KB];
+  };
+  volatile float rmem[RMEM ? CT * (2 + 4 * KB) : 1];
+  auto qmem = []() __attribute__((always_inline)) -> uint4* {
+    if constexpr (QLDS) {
+      __shared__ uint4 q[CT * kWaves * KB * 64];
+      return q;
+    }
+    return nullptr;
+  };
+  Run rreg[CT];
+  auto run_get = [&](int ct, bool first, Run& r) __attribute__((always_inline)) {
+    if (SEG != SEG_WALK || first) {  // the fold of the first segment leaves it as it is
+      r.R = -FLT_MAX;
+      r.S = 0.f;
+#pragma unroll
+      for (int k = 0; k < KB; k++) r.Q[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    } else if constexpr (RMEM) {
+      r.R = rmem[ct * (2 + 4 * KB)];
+      r.S = rmem[ct * (2 + 4 * KB) + 1];
+#pragma unroll
+      for (int k = 0; k < KB; k++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) r.Q[k][e] = rmem[ct * (2 + 4 * KB) + 2 + 4 * k + e];
+    } else if constexpr (QLDS) {
+      r.R = rreg[ct].R;
+      r.S = rreg[ct].S;
+#pragma unroll
+      for (int k = 0; k < KB; k++)
+        r.Q[k] = __builtin_bit_cast(f32x4_t, ld16(qmem() + ((ct * kWaves + wave) * KB + k) * 64 + lane));
+    } else {
+      r = rreg[ct];
+    }
+  };
+  auto run_put = [&](int ct, const Run& r) __attribute__((always_inline)) {
+    if constexpr (RMEM) {
+      rmem[ct * (2 + 4 * KB)] = r.R;
+      rmem[ct * (2 + 4 * KB) + 1] = r.S;
+#pragma unroll
+      for (int k = 0; k < KB; k++)
+#pragma unroll
+        for (int e = 0; e < 4; e++) rmem[ct * (2 + 4 * KB) + 2 + 4 * k + e] = r.Q[k][e];
+    } else if constexpr (QLDS) {
+      rreg[ct].R = r.R;
+      rreg[ct].S = r.S;
+#pragma unroll
+      for (int k = 0; k < KB; k++)
+        st16(qmem() + ((ct * kWaves + wave) * KB + k) * 64 + lane, __builtin_bit_cast(uint4, r.Q[k]));
+    } else {
+      rreg[ct] = r;
+    }
+  };
+  static_assert(CT <= 2, "running state of one or two column tiles");
+  // A segment's end inside the walk: the chains exchange (m, l, o) through
+  // this wave's part of value slot `slot`, whose block has been used and
+  // whose refill the caller orders behind the readers; the loads of the next
+  // blocks stay in flight (asm LDS accesses, see ds_read_tr).
+  auto mls = []() __attribute__((always_inline)) -> float2* {
+    if constexpr (!KL && SEG == SEG_WALK) {
+      __shared__ float2 ml[kWaves * 16];
+      return ml;
+    }
+    return nullptr;
+  };
+  auto mid_merge = [&](int slot, bool first) __attribute__((always_inline)) {
+    const uint32_t ob = (uint32_t)(uintptr_t)(lds_void_t*)(arr(slot) + C::KSLOT) + lane * 16;
+    // (m, l) of a column, which its four lanes all hold.
+    const uint32_t mb = KL ? (uint32_t)(uintptr_t)(lds_void_t*)arr(slot) + r16 * 8
+                           : (uint32_t)(uintptr_t)(lds_void_t*)mls() + r16 * 8;
+    constexpr uint32_t MS = KL ? C::VSLOT * 16 : 16 * 8;  // bytes between the chains' (m, l)
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) {
+      if (ct > 0) asm volatile("s_barrier" ::: "memory");  // the last tile's readers
+#pragma unroll
+      for (int db = 0; db < NB; db++) ds_write_acc(ob + (wslot + db * 64) * 16, o[ct][db]);
+      const f32x2_t mv = {m[ct], l[ct]};
+      asm volatile("ds_write_b64 %0, %1" ::"v"(mb + wave * MS), "v"(mv) : "memory");
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      u32x2_t sv[kWaves];
+      u32x4_t ov[KB][kWaves];
+#pragma unroll
+      for (int c = 0; c < kWaves; c++)
+        asm volatile("ds_read_b64 %0, %1" : "=v"(sv[c]) : "v"(mb + c * MS) : "memory");
+#pragma unroll
+      for (int k = 0; k < KB; k++) {
+        const int db = wave + kWaves * k < NB ? wave + kWaves * k : 0;
+#pragma unroll
+        for (int c = 0; c < kWaves; c++) ov[k][c] = ds_read_b128(ob + (c * C::VSLOT + db * 64) * 16);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int c = 0; c < kWaves; c++) {
+        asm volatile("" : "+v"(sv[c]));
+#pragma unroll
+        for (int k = 0; k < KB; k++) asm volatile("" : "+v"(ov[k][c]));
+      }
+      float ec[kWaves];
+      const float sk = first && p.sinks ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e
+                                        : -FLT_MAX;
+      float M = sk;
+#pragma unroll
+      for (int c = 0; c < kWaves; c++) M = fmaxf(M, __uint_as_float(sv[c][0]));
+      float L = first && p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
+#pragma unroll
+      for (int c = 0; c < kWaves; c++) {
+        ec[c] = __builtin_amdgcn_exp2f(__uint_as_float(sv[c][0]) - M);
+        L = __builtin_fmaf(__uint_as_float(sv[c][1]), ec[c], L);
+      }
+      Run r;
+      run_get(ct, first, r);
+      const FoldW w = fold_stats(r.R, r.S, M, L);
+#pragma unroll
+      for (int k = 0; k < KB; k++) {
+        f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < kWaves; c++) {
+          const f32x4_t oc = __builtin_bit_cast(f32x4_t, ov[k][c]);
+#pragma unroll
+          for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
+        }
+        fold_out(r.Q[k], O, w);
+      }
+      run_put(ct, r);
+      m[ct] = -FLT_MAX;
+      l[ct] = 0.f;
+#pragma unroll
+      for (int i = 0; i < NB; i++) o[ct][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+
   // Block i of the chain: keys loaded at step i - PK, values at step
   // i - SV + 1 into slot i % SV. The loop is unrolled over U steps (the
   // least common multiple of the two rotations) so that register and slot
@@ -791,7 +967,11 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
           // their latency.
           VA_t va;
           vread((u + SV - 1) % SV, va);
-          update(std::true_type{}, sp, kr[0].m, (u + SV - 1) % SV, wave + kWaves * (j - 1), va);
+          update(std::true_type{}, sp, kr[0].m, (u + SV - 1) % SV, blk0 + wave + kWaves * (j - 1), va);
+        }
+        // (Barrier j + 1 precedes the slot's refill.)
+        if constexpr (SEG == SEG_WALK) {
+          if (ends_segment(j)) mid_merge((u + SV - 1) % SV, j == kSegIt);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         scores(kr[0], kl, sp);
@@ -805,7 +985,10 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
         const int j = j0 + u;
         if (j >= steps) break;
         asm volatile("s_barrier" ::: "memory");
-        if (j < nit) compute(kr[0], kr[0].m, u, wave + kWaves * j);
+        if (j < nit) compute(kr[0], kr[0].m, u, blk0 + wave + kWaves * j);
+        if constexpr (SEG == SEG_WALK) {  // (barrier j + 1 precedes the slot's refill)
+          if (ends_segment(j + 1)) mid_merge(u, j + 1 == kSegIt);
+        }
       }
     }
   } else {
@@ -813,7 +996,8 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
     for (int u = 0; u < SV - 1; u++) ld.vload(u, arr(u) + wslot);
 #pragma unroll
     for (int u = 0; u < PK; u++) ld.kload(u, kr[u]);
-    for (int i0 = 0; i0 < nit; i0 += U) {
+    static_assert(kSegIt % U == 0, "segments end on a round of the loop");
+    for (int i0 = 0; i0 < (SEG == SEG_WALK ? nit0 : nit); i0 += U) {
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int i = i0 + u;
@@ -822,17 +1006,21 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
         ld.vload(i + SV - 1, arr((u + SV - 1) % SV) + wslot);
         if (i < nit) {
           if constexpr (MK == 2)
-            compute(kr[u % (PK + 1)], mcur.m, u % SV, wave + kWaves * i);
+            compute(kr[u % (PK + 1)], mcur.m, u % SV, blk0 + wave + kWaves * i);
           else
-            compute(kr[u % (PK + 1)], kr[u % (PK + 1)].m, u % SV, wave + kWaves * i);
+            compute(kr[u % (PK + 1)], kr[u % (PK + 1)].m, u % SV, blk0 + wave + kWaves * i);
+        }
+        if (SEG == SEG_WALK && u == U - 1 && ends_segment(i + 1)) {
+          mid_merge(u % SV, i + 1 == kSegIt);
+          asm volatile("s_barrier" ::: "memory");  // the slot's readers, before its refill
         }
       }
     }
   }
 
-  // Merge the 4 chains in order through LDS, one column tile at a time: o of
-  // chain c in va0, (m, l) in va1 (the value slots are free once every
-  // wave's loads and reads have completed).
+  // The last segment's merge, one column tile at a time: o of chain c in va0,
+  // (m, l) in va1 (the value slots are free once every wave's loads and reads
+  // have completed); then its fold and the output, or the partial result.
   uint4* const mo = va0;
   float2* const ml = reinterpret_cast<float2*>(va1);
 #pragma unroll
@@ -847,7 +1035,8 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
     asm volatile("s_barrier" ::: "memory");
     float mc[kWaves], lc[kWaves], ec[kWaves];
     // The sink (base 2) first: -FLT_MAX without one.
-    const float sk = p.sinks ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e : -FLT_MAX;
+    const bool sink = p.sinks && (SEG == SEG_ONE || (SEG == SEG_WALK ? nsg <= 1 : seg == 0));
+    const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e : -FLT_MAX;
     float M = sk;
 #pragma unroll
     for (int c = 0; c < kWaves; c++) {
@@ -856,17 +1045,29 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
       lc[c] = v.y;
       M = fmaxf(M, mc[c]);
     }
-    float L = p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
+    float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
 #pragma unroll
     for (int c = 0; c < kWaves; c++) {
       ec[c] = __builtin_amdgcn_exp2f(mc[c] - M);
       L = __builtin_fmaf(lc[c], ec[c], L);
     }
-    T* __restrict__ out =
-        static_cast<T*>(p.out) + ((b * p.H + head[ct]) * p.qL + srow[ct]) * V + ws * C::DW;
+    const int64_t col = (b * p.H + head[ct]) * p.qL + srow[ct];
+    Run r;
+    FoldW w = {0.f, 0.f};
+    if constexpr (SEG == SEG_WALK) {
+      run_get(ct, nsg <= 1, r);
+      w = fold_stats(r.R, r.S, M, L);
+      L = r.S;
+    }
+    if constexpr (SEG == SEG_SPLIT) {
+      if (colv[ct] && ws == 0 && wave == 0 && g == 0)
+        *reinterpret_cast<float2*>(p.part + p.B * p.H * p.qL * p.nseg * V + (col * p.nseg + seg) * 2) =
+            make_float2(M, L);
+    }
+    T* __restrict__ out = static_cast<T*>(p.out) + col * V + ws * C::DW;
     // Wave w writes out the dim blocks w, w + 4, ... of this workgroup.
 #pragma unroll
-    for (int k = 0; k < (NB + kWaves - 1) / kWaves; k++) {
+    for (int k = 0; k < KB; k++) {
       const int db = wave + kWaves * k;
       if (db >= NB) break;
       f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -876,14 +1077,34 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
 #pragma unroll
         for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
       }
-      unsigned short ob[4];
+      if constexpr (SEG == SEG_SPLIT) {
+        float* __restrict__ part = p.part + (col * p.nseg + seg) * V + ws * C::DW;
+        if (colv[ct]) *reinterpret_cast<f32x4_t*>(part + 16 * db + 4 * g) = O;
+      } else {
+        if constexpr (SEG == SEG_WALK) {
+          fold_out(r.Q[k], O, w);
+          O = r.Q[k];
+        }
+        unsigned short ob[4];
 #pragma unroll
-      for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
-      if (colv[ct])
-        *reinterpret_cast<uint2*>(out + 16 * db + 4 * g) =
-            make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
+        for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
+        if (colv[ct])
+          *reinterpret_cast<uint2*>(out + 16 * db + 4 * g) =
+              make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
+      }
     }
   }
+}
+
+template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
+__global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs p) {
+  sdpa_mfma_body<T, D, V, CT, PK, SV, WS, MK, KL, LW, SEG>(p);
+}
+// The same with the registers of as many waves per SIMD (two, or three for
+// heads up to 64) as the two-tile kernels of one segment leave room for.
+template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
+__global__ void __launch_bounds__(kThreads + 64 * LW, D + V <= 128 ? 3 : 2) sdpa_mfma_kernel2(SdpaArgs p) {
+  sdpa_mfma_body<T, D, V, CT, PK, SV, WS, MK, KL, LW, SEG>(p);
 }
 
 // f(integral_constant<I>) for I = I0 .. N - 1 while it returns true.
@@ -1004,12 +1225,13 @@ struct Shared {
   };
 };
 
-template <typename T, int D, int V, int NW, int GP, int NG>
+template <typename T, int D, int V, int NW, int GP, int NG, int SEG>
 __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
   using C = Shared<T, D, V, NW, GP, NG>;
   constexpr int NQ = C::NQ, NB = C::NB, CH = C::CH, VCH = C::VCH, LPW = C::LPW;
   constexpr int COLS = 16 * NW;  // columns per workgroup
   __shared__ uint4 ring[C::S * C::SLOT];
+
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1250,23 +1472,84 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
     static_for<0, GP>(blockstep);
     return true;
   };
+  // SEG_WALK: the running state (R, S, Q) over the segments so far; Q in LDS
+  // (in registers it would not fit beside the 4 chains' state).
+  float R = -FLT_MAX, S = 0.f;
+  bool folded = false;
+  auto run_lds = []() __attribute__((always_inline)) -> uint4* {
+    if constexpr (SEG == SEG_WALK) {
+      __shared__ uint4 run[NW * NB * 64];
+      return run;
+    }
+    return nullptr;
+  };
+  static_assert(kSegBlk % (UG * GP) == 0, "segments end on a round of the loop");
+  if constexpr (SEG == SEG_WALK) {
+    // Every segment but the last: its blocks, then, for a wave whose columns
+    // see keys past it, its chains merge and fold.
+    for (int end = kSegBlk; end < nblk; end += kSegBlk) {
+      for (; q0 * GP < end; q0 += UG) static_for<0, UG>(group);
+      if (end < nvis_w) {
+        const bool sink = p.sinks && !folded;
+        const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
+        float M = sk;
+#pragma unroll
+        for (int c = 0; c < 4; c++) M = fmaxf(M, m[c]);
+        float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
+        float ec[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          ec[c] = __builtin_amdgcn_exp2f(m[c] - M);
+          L = __builtin_fmaf(l[c], ec[c], L);
+        }
+        const FoldW w = fold_stats(R, S, M, L);
+        uint4* const run = run_lds() + wave * NB * 64 + lane;
+#pragma unroll
+        for (int db = 0; db < NB; db++) {
+          f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int c = 0; c < 4; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(o[c][db][e], ec[c], O[e]);
+          f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
+          if (folded) Q = __builtin_bit_cast(f32x4_t, ld16(run + db * 64));  // wave-uniform
+          fold_out(Q, O, w);
+          st16(run + db * 64, __builtin_bit_cast(uint4, Q));
+        }
+        folded = true;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          m[c] = -FLT_MAX;
+          l[c] = 0.f;
+#pragma unroll
+          for (int i = 0; i < NB; i++) o[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        }
+      }
+    }
+  }
   for (; q0 * GP < nblk; q0 += UG) static_for<0, UG>(group);
   // The loads issued past the last block (they read nothing but still write
   // their slots) complete before the workgroup's LDS is released.
   __builtin_amdgcn_s_waitcnt(kWaitAll);
 
-  // Merge the 4 chains in order, in registers (the sink first: -FLT_MAX
-  // without one).
-  const float sk = p.sinks ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
+  // Merge the 4 chains in order, in registers (the sink first, in the first
+  // segment: -FLT_MAX without one).
+  const bool sink = SEG == SEG_ONE ? p.sinks != nullptr : p.sinks && !folded;
+  const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
   float M = sk;
 #pragma unroll
   for (int c = 0; c < 4; c++) M = fmaxf(M, m[c]);
-  float L = p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
+  float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
   float ec[4];
 #pragma unroll
   for (int c = 0; c < 4; c++) {
     ec[c] = __builtin_amdgcn_exp2f(m[c] - M);
     L = __builtin_fmaf(l[c], ec[c], L);
+  }
+  FoldW w = {0.f, 0.f};
+  if constexpr (SEG == SEG_WALK) {
+    w = fold_stats(R, S, M, L);
+    L = S;
   }
   T* __restrict__ out = static_cast<T*>(p.out) + ((b * p.H + head) * p.qL + srow) * V;
 #pragma unroll
@@ -1276,6 +1559,12 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
     for (int c = 0; c < 4; c++)
 #pragma unroll
       for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(o[c][db][e], ec[c], O[e]);
+    if constexpr (SEG == SEG_WALK) {
+      f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      if (folded) Q = __builtin_bit_cast(f32x4_t, ld16(run_lds() + (wave * NB + db) * 64 + lane));
+      fold_out(Q, O, w);
+      O = Q;
+    }
     unsigned short ob[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
@@ -1298,50 +1587,63 @@ constexpr int sdpa_loader_slots(int D, int V, int WS) {
 // through LDS by contiguous loads (sdpa_loader_slots). Wide heads (D or V above
 // 128) load no keys ahead. Keys one block ahead and values in two slots
 // otherwise: deeper prefetch measured no faster.
-template <typename T, int D, int V, bool MASK, int SHAPE>
+template <typename T, int D, int V, bool MASK, int SHAPE, int SEG>
 constexpr SdpaKernelFn mfma_kernel() {
   constexpr int MK = MASK ? 1 : 0;
   constexpr int PK = sdpa_wide(D, V) ? 0 : 1;
   constexpr int WS = sdpa_shape_splits(V, SHAPE);
   if constexpr (SHAPE == SDPA_SHARED) {
-    if constexpr (sdpa_shared_dims(D, V) && !MASK)
-      return sdpa_shared_kernel<T, D, V, sdpa_shared_waves(D, V), 2, 2>;
+    if constexpr (sdpa_shared_dims(D, V) && !MASK && SEG != SEG_SPLIT)
+      return sdpa_shared_kernel<T, D, V, sdpa_shared_waves(D, V), 2, 2, SEG>;
     else
       return nullptr;
   } else if constexpr (SHAPE == SDPA_ROWS) {
-    return sdpa_mfma_kernel<T, D, V, sdpa_rows_tiles(D, V), MASK ? 0 : PK, 2, WS, MASK ? 2 : 0,
-                            false, 0>;
+    constexpr int CT = sdpa_rows_tiles(D, V);
+    if constexpr (CT == 2 && SEG == SEG_WALK)
+      return sdpa_mfma_kernel2<T, D, V, CT, MASK ? 0 : PK, 2, WS, MASK ? 2 : 0, false, 0, SEG>;
+    else
+      return sdpa_mfma_kernel<T, D, V, CT, MASK ? 0 : PK, 2, WS, MASK ? 2 : 0, false, 0, SEG>;
   } else if constexpr (SHAPE == SDPA_TILE) {
-    return sdpa_mfma_kernel<T, D, V, 1, PK, 2, WS, MK, false, 0>;
+    return sdpa_mfma_kernel<T, D, V, 1, PK, 2, WS, MK, false, 0, SEG>;
   } else {
     // Keys in LDS with loader waves (sdpa_loaders: the host launches 8 waves).
     constexpr bool KLS = sdpa_loaders(D, V, SHAPE, MASK);
     return sdpa_mfma_kernel<T, D, V, 1, KLS ? 0 : PK, KLS ? sdpa_loader_slots(D, V, WS) : 2, WS, MK, KLS,
-                            KLS ? kWaves : 0>;
+                            KLS ? kWaves : 0, SEG>;
   }
 }
 
+template <typename T, int D, int V, bool MASK, int SHAPE>
+SdpaKernelFn mfma_kernel_seg(int seg) {
+  switch (seg) {
+    case SEG_ONE: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_ONE>();
+    case SEG_WALK: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_WALK>();
+    case SEG_SPLIT: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_SPLIT>();
+  }
+  return nullptr;
+}
+
 template <typename T, int D, int V, bool MASK>
-SdpaKernelFn mfma_kernel_shape(int shape) {
+SdpaKernelFn mfma_kernel_shape(int shape, int seg) {
   switch (shape) {
-    case SDPA_ROWS: return mfma_kernel<T, D, V, MASK, SDPA_ROWS>();
-    case SDPA_TILE: return mfma_kernel<T, D, V, MASK, SDPA_TILE>();
-    case SDPA_SPLIT2: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT2>();
-    case SDPA_SPLIT4: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT4>();
-    case SDPA_SPLIT8: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT8>();
-    case SDPA_SHARED: return mfma_kernel<T, D, V, MASK, SDPA_SHARED>();
+    case SDPA_ROWS: return mfma_kernel_seg<T, D, V, MASK, SDPA_ROWS>(seg);
+    case SDPA_TILE: return mfma_kernel_seg<T, D, V, MASK, SDPA_TILE>(seg);
+    case SDPA_SPLIT2: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT2>(seg);
+    case SDPA_SPLIT4: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT4>(seg);
+    case SDPA_SPLIT8: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT8>(seg);
+    case SDPA_SHARED: return mfma_kernel_seg<T, D, V, MASK, SDPA_SHARED>(seg);
   }
   return nullptr;
 }
 
 template <int D, int V>
-SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape) {
+SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape, int seg) {
   if (dtype == BI_BF16)
-    return mask ? mfma_kernel_shape<__bf16, D, V, true>(shape)
-                : mfma_kernel_shape<__bf16, D, V, false>(shape);
+    return mask ? mfma_kernel_shape<__bf16, D, V, true>(shape, seg)
+                : mfma_kernel_shape<__bf16, D, V, false>(shape, seg);
   if (dtype == BI_F16)
-    return mask ? mfma_kernel_shape<_Float16, D, V, true>(shape)
-                : mfma_kernel_shape<_Float16, D, V, false>(shape);
+    return mask ? mfma_kernel_shape<_Float16, D, V, true>(shape, seg)
+                : mfma_kernel_shape<_Float16, D, V, false>(shape, seg);
   return nullptr;
 }
 
@@ -1349,7 +1651,7 @@ SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape) {
 
 // Defines the lookup of one head-dim pair's kernels (declared in
 // bi_sdpa_args.h); each instantiation unit expands it once.
-#define BI_SDPA_MFMA_DEFINE(D, V)                                                   \
-  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape) {      \
-    return mfma_kernel_for<D, V>(dtype, mask, shape);                               \
+#define BI_SDPA_MFMA_DEFINE(D, V)                                                        \
+  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int seg) {  \
+    return mfma_kernel_for<D, V>(dtype, mask, shape, seg);                               \
   }

@@ -5,12 +5,13 @@ normalisation, validation, sinks, launch) on top of the HIP kernels in
 csrc/ (bi_sdpa.hip: fp32 on the vector ALUs; bi_sdpa_mfma_kernel.h: bf16 and
 f16 on matrix cores), reached through the C ABI ``bi_sdpa`` (include/bi.h).
 
-One workgroup owns the entire reduction over the keys for each of its query
-rows. fp32 splits it into 32 partial online softmaxes by key index (key i
-belongs to partial i mod 32); bf16/f16 into 4 chains of 32-key blocks (block b
-belongs to chain b mod 4); the partials are combined in a fixed order. Nothing
-in that order depends on the number of query rows, the batch, or how far the
-key sequence extends past the keys a row can see.
+fp32 splits a query row's reduction over the keys into 32 partial online
+softmaxes by key index (key i belongs to partial i mod 32) in one workgroup;
+bf16/f16 into segments of 2048 keys at fixed positions, each into 4 chains of
+32-key blocks (block b belongs to chain b mod 4), in one workgroup or, for
+grids that would leave the GPU idle, one per segment. The partials are combined
+in a fixed order. Nothing in that order depends on the number of query rows,
+the batch, or how far the key sequence extends past the keys a row can see.
 """
 
 import ctypes
@@ -97,9 +98,11 @@ def _sdpa(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks):
     return _sdpa_eager(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks)
 
 
-def _sdpa_eager(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks, shape=None):
+def _sdpa_eager(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks, shape=None,
+                split=False):
     """The launch; `shape` forces a launch shape (bi_sdpa_with_shape,
-    include/bi_testing.h) instead of the one bi_sdpa picks."""
+    include/bi_testing.h) instead of the one bi_sdpa picks, `split` one segment
+    of the keys per workgroup in it (bi_sdpa_split_with_shape)."""
     B, H, qL, D = q.shape
     _, Hkv, N, _ = k.shape
     V = v.shape[-1]
@@ -117,18 +120,33 @@ def _sdpa_eager(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks,
             B, H, Hkv, qL, N, D, V, strides, float(scale), int(mask_mode),
             int(causal_offset), _lib.DTYPE_CODES[q.dtype])
     stream, switch = _lib.launch_stream(q.device)
-    if shape is None:
-        fn, tail = L.bi_sdpa, (stream,)
-    else:
-        fn, tail = L.bi_sdpa_with_shape, (int(shape), stream)
     if switch:
         with torch.cuda.device(q.device):
-            rc = fn(*args, *tail)
+            rc = _launch(L, args, shape, split, q, stream)
     else:
-        rc = fn(*args, *tail)
+        rc = _launch(L, args, shape, split, q, stream)
     if rc:
         _lib.check(rc, "bi_sdpa")
     return out
+
+
+def _launch(L, args, shape, split, q, stream):
+    B, H, Hkv, qL, N, D, V = args[7:14]
+    if shape is not None and not split:
+        return L.bi_sdpa_with_shape(*args, int(shape), stream)
+    need = 0
+    if split:
+        need = B * H * qL * -(-N // _lib.SDPA_SEGMENT) * (V + 2) * 4
+    elif N > _lib.SDPA_SEGMENT:
+        need = L.bi_sdpa_workspace(B, H, Hkv, qL, N, D, V, args[18], args[16])
+    if not need:
+        return L.bi_sdpa(*args, stream)
+    # Used by this stream's launches only, so the caching allocator may give
+    # it to the next call on the stream as soon as it is dropped here.
+    ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+    if split:
+        return L.bi_sdpa_split_with_shape(*args, int(shape), ws.data_ptr(), need, stream)
+    return L.bi_sdpa_ws(*args, ws.data_ptr(), need, stream)
 
 
 def launch_shape(q, k, v, mask_mode=_lib.MASK_NONE):

@@ -36,6 +36,11 @@ SIGNATURES = {
     "bi_sdpa": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64p, _c_vp, _c_vp,
                          _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                          _c_i64p, _c_float, _c_int, _c_i64, _c_int, _c_vp]),
+    "bi_sdpa_workspace": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                   _c_int, _c_int]),
+    "bi_sdpa_ws": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64p, _c_vp, _c_vp,
+                            _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                            _c_i64p, _c_float, _c_int, _c_i64, _c_int, _c_vp, _c_i64, _c_vp]),
     "bi_gemm_num_geometries": (_c_int, []),
     "bi_gemm_geometry_info": (_c_int, [_c_int, ctypes.POINTER(_c_int), ctypes.POINTER(_c_int),
                                        ctypes.POINTER(_c_int)]),
@@ -58,12 +63,17 @@ SIGNATURES = {
     "bi_sdpa_with_shape": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64p, _c_vp, _c_vp,
                                     _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
                                     _c_i64p, _c_float, _c_int, _c_i64, _c_int, _c_int, _c_vp]),
+    "bi_sdpa_split_with_shape": (_c_int, [_c_vp, _c_vp, _c_vp, _c_vp, _c_i64p, _c_vp, _c_vp,
+                                          _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
+                                          _c_i64p, _c_float, _c_int, _c_i64, _c_int, _c_int,
+                                          _c_vp, _c_i64, _c_vp]),
     "bi_device_wavefront_size": (_c_int, [ctypes.POINTER(_c_int)]),
 }
 
 # Attention launch shapes (include/bi_testing.h): bf16 / f16 on matrix cores.
 SDPA_ROWS, SDPA_TILE, SDPA_SPLIT2, SDPA_SPLIT4, SDPA_SPLIT8, SDPA_SHARED = 0, 1, 2, 3, 4, 5
 SDPA_NUM_SHAPES = 6
+SDPA_SEGMENT = 2048  # keys per segment of the bf16/f16 kernels (bi_sdpa_args.h kSegKeys)
 
 ABI_VERSION = 1
 

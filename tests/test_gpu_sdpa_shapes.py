@@ -29,7 +29,7 @@ import torch
 from mlx_batch_invariant import _attention, _lib
 from oracle import sdpa as osdpa
 
-from helpers import bits, f64, rn
+from helpers import bits, f64, ndiff, rn
 
 pytestmark = pytest.mark.gpu
 
@@ -477,3 +477,59 @@ def test_fp32_head_grouping_prefill(cuda):
         for s in (0, 17, qL - 1):
             alone = _alone(q, k, v, spec, 0, s)
             assert np.array_equal(bits(alone[0, :, 0]), bits(y[0, :, s])), s
+
+
+@pytest.mark.parametrize("D,V", [(128, 128), (64, 64), (256, 256), (576, 512)])
+@pytest.mark.parametrize("N", [2047, 2049, 4096, 6200])
+def test_segments_give_the_same_bits_in_one_workgroup_or_each_in_its_own(cuda, D, V, N):
+    """bf16 / f16: past one segment of keys, every launch shape that walks all
+    segments and every one that takes one segment per workgroup, with a second
+    kernel folding them, gives the same bits: without a mask, causal with
+    sinks, and with an additive mask that hides the whole first or last
+    segment from some rows; rows against float64."""
+    H, Hkv, qL, B = 8, 2, 5, 2
+    for dname, dtype in (("float16", torch.float16), ("bfloat16", torch.bfloat16)):
+        q = rn((B, H, qL, D), dtype, 71, device=cuda)
+        k = rn((B, Hkv, N, D), dtype, 72, device=cuda)
+        v = rn((B, Hkv, N, V), dtype, 73, device=cuda)
+        sinks = rn((H,), dtype, 74, std=3.0, device=cuda)
+        add = rn((B, 1, qL, N), dtype, 75, device=cuda)
+        add[:, :, 0, :2048] = -float("inf")
+        add[:, :, 1, -(N % 2048 or 2048):] = -float("inf")
+        for mode, mask, ms, sk in ((0, None, (0, 0, 0), None), (1, None, (0, 0, 0), sinks),
+                                   (2, add, (qL * N, 0, N), None)):
+            outs = {}
+            for shape in range(_lib.SDPA_NUM_SHAPES):
+                for split in (False, True):
+                    try:
+                        outs[shape, split] = _attention._sdpa_eager(
+                            q, k, v, D ** -0.5, mode, mask, ms, N - qL, sk, shape=shape, split=split)
+                    except (ValueError, NotImplementedError):
+                        # "shared" takes D = V <= 128 without an array mask, and has no split form.
+                        assert shape == _lib.SDPA_SHARED
+            base = outs[_lib.SDPA_TILE, False]
+            for key, y in outs.items():
+                assert ndiff(y, base) == 0, "%s N=%d mode %d shape %d split %s" % (
+                    dname, N, mode, key[0], key[1])
+            picked = _attention._sdpa_eager(q, k, v, D ** -0.5, mode, mask, ms, N - qL, sk)
+            assert ndiff(picked, base) == 0
+            bias = None if mask is None else f64(mask)
+            if mode == 1:
+                vis = np.arange(N)[None, :] <= np.arange(qL)[:, None] + N - qL
+                bias = np.where(vis, 0.0, -np.inf)[None, None]
+            kk, vv = (np.repeat(f64(t), H // Hkv, axis=1) for t in (k, v))
+            s = np.einsum("bhqd,bhnd->bhqn", f64(q), kk) * D ** -0.5
+            s = s if bias is None else s + bias
+            top = s.max(-1, keepdims=True)
+            if sk is not None:
+                top = np.maximum(top, f64(sk)[None, :, None, None])
+            top = np.maximum(top, -1e30)  # a row whose keys are all hidden is 0
+            p = np.exp(s - top)
+            den = p.sum(-1, keepdims=True)
+            if sk is not None:
+                den = den + np.exp(f64(sk)[None, :, None, None] - top)
+            want = np.einsum("bhqn,bhnd->bhqd", p / np.maximum(den, 1e-300), vv)
+            # p and the output round once each to the element type (relative
+            # 2^-9 bf16, 2^-12 f16, per product of the sum): 2-norm within 2.5 of it.
+            err = np.linalg.norm(f64(base) - want) / np.linalg.norm(want)
+            assert err < 2.5 * 2.0 ** (-9 if dname == "bfloat16" else -12), (dname, N, mode, err)
