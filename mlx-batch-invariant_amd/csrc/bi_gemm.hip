@@ -140,8 +140,11 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
 // Id of the quantized decode footprint (bi_gemm_qdecode.h: 2-, 4- or 8-bit
 // codes, at most 8 rows), one past the dense table.
 constexpr int kQDecode = kNumGeometries;
+// The quantized prefill footprint: whole stages of K only.
+constexpr int kQPrefill = 8;
+constexpr int kQPrefillStage = 64;
 
-int pick_qgeometry(int64_t M, int64_t N, int64_t K, int bits) {
+int pick_qgeometry(int64_t M, int64_t N, int64_t K, int bits, int group) {
   // The decode footprint. 2- and 4-bit: up to 4 rows everywhere; 5-8 rows
   // (an LDS share and register count that fit one workgroup per CU) only
   // while the column blocks fit one round over the 256 CUs (4-bit, N = 4096,
@@ -163,7 +166,25 @@ int pick_qgeometry(int64_t M, int64_t N, int64_t K, int bits) {
     if (t128 >= 160) return 3;
     return t64 >= 192 ? 2 : 5;
   }
-  return (M <= 256 ? t128 : ceil_div(N, 128)) >= 200 ? 3 : 2;
+  if (M <= 256 || K % kQPrefillStage)
+    return (M <= 256 ? t128 : ceil_div(N, 128)) >= 200 ? 3 : 2;
+  // More rows: 64 x 64 tiles or the prefill footprint's 128 x 64, whichever
+  // has the less estimated time: rounds of 256 workgroups times a round's
+  // (4-bit, K = 4096, in 0.1 us; the prefill footprint's first takes longer,
+  // one workgroup alone on a CU). Group 64: M = 1024, N = 11008 188 us in 64 x
+  // 64 tiles, 162 in 128 x 64; M = 512, N = 4096 40 and 46; M = 2048, N = 4096
+  // 140 and 120. Group 32: M = 1024, N = 11008 256 and 215. Group 128: 174 and
+  // 175, N = 32000 492 and 465.
+  const int64_t small = group == 32 ? 233 : group == 64 ? 173 : 158;
+  const int64_t large = group == 32 ? 355 : group == 64 ? 280 : 295;
+  const int64_t first = group == 32 ? 590 : 465;
+  const int64_t t_small = std::max<int64_t>(ceil_div(t64, 256), 2) * small;
+  const int64_t n_large = ceil_div(ceil_div(M, 128) * ceil_div(N, 64), 256);
+  // Two workgroups fit a CU for groups 32 and 128 (three for 64): an odd third
+  // round runs alone.
+  const int64_t extra = n_large == 2 ? large / 8 : n_large == 3 && group != 64 ? large / 2 : 0;
+  const int64_t t_large = std::max(n_large * large + extra, first);
+  return t_large < t_small ? kQPrefill : 2;
 }
 
 int validate(const void* a, const void* b, void* out, int64_t M, int64_t N, int64_t K,
@@ -483,6 +504,9 @@ int qlaunch(const void* x, const void* w, const void* scales, const void* biases
     return qlaunch_decode(x, w, scales, biases, out, M, N, K, group_size, bits, dtype, stream);
   const Geometry& G = kGeometries[g];
   const int64_t lim = (int64_t)1 << 31;
+  if (g == kQPrefill && (K == 0 || K % kQPrefillStage))
+    return bi::fail(BI_EUNSUPPORTED, "bi_qgemm: geometry %d takes K in multiples of %d only", g,
+                    kQPrefillStage);
   if ((int64_t)G.bm * K * 2 >= lim || (int64_t)G.bn * K * bits / 8 >= lim)
     return bi::fail(BI_EUNSUPPORTED, "bi_qgemm: operand panel of 2 GiB or more");
   GemmArgs p = {};
@@ -519,7 +543,7 @@ extern "C" int bi_qgemm(const void* x, const void* w, const void* scales, const 
   const int rc = qvalidate(x, w, scales, biases, out, M, N, K, group_size, bits, dtype);
   if (rc != BI_OK || M == 0 || N == 0) return rc;
   return qlaunch(x, w, scales, biases, out, M, N, K, group_size, bits, dtype,
-                 pick_qgeometry(M, N, K, bits), hip_stream);
+                 pick_qgeometry(M, N, K, bits, group_size), hip_stream);
 }
 
 extern "C" int bi_qgemm_num_geometries(void) { return kQDecode + 1; }
@@ -527,7 +551,7 @@ extern "C" int bi_qgemm_num_geometries(void) { return kQDecode + 1; }
 extern "C" int bi_qgemm_pick_geometry(int64_t M, int64_t N, int64_t K, int bits) {
   if (bits != 2 && bits != 4 && bits != 8)
     return bi::fail(BI_EINVAL, "bi_qgemm: bits must be 2, 4 or 8, got %d", bits);
-  return pick_qgeometry(M, N, K, bits);
+  return pick_qgeometry(M, N, K, bits, 64);
 }
 
 extern "C" int bi_qgemm_with_geometry(const void* x, const void* w, const void* scales,

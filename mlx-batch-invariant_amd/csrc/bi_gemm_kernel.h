@@ -353,8 +353,9 @@ struct Slot {
 struct QSlot {
   uint4* a;
   uint4* b;
-  unsigned short* s16;
+  unsigned short* s16;  // element bits, or
   unsigned short* z16;
+  float2* sz;           // (QF32) as fp32
 };
 
 template <typename T, int BM, int BN, int WM, int WN, int NW, int KB, int NS, bool TB, int QB = 0,
@@ -976,12 +977,29 @@ struct GemmTile {
   // layout) from +0.0. That is sum_k x_k * (scale * q_k + bias) with fp32
   // roundings only -- the reference's fp32 product with its fp32 weights to
   // within fp32 accumulation error -- and a fixed sequence per output element.
-  static constexpr int QP = NW == 8 ? 2 : 4;  // stages of loads in flight (registers)
+  static constexpr int QP = NW == 8 || (BM == 128 && BN == 64) ? 2 : 4;  // stages of loads in flight (registers)
   // Threads that load and stage the quantized operands: the waves that do
   // not compute, when there are such (the computing waves then only read LDS
   // and run the MFMAs and folds), else all.
   static constexpr int QNT = (QB != 0 && NW > CW) ? 64 * (NW - CW) : NT;
   static constexpr int QLA = (A_CH + QNT - 1) / QNT;
+  // The prefill footprint, 128 x 64 by four waves: the A tile goes straight to
+  // LDS, one stage ahead, and stages are whole, so a wave keeps 136-144
+  // registers (group 64; 172-196 for 32 and 128) and three (two) workgroups
+  // share a CU where 128 x 128 tiles by eight waves of 180-221 ran alone, two
+  // waves a SIMD with nothing to do at every barrier and a last round of
+  // tiles twice as long. Bound by issue: a stage is 20 MFMAs and 64 fused
+  // multiply-adds of the fold per wave, which a SIMD does not overlap, and 24
+  // other vector instructions. 4-bit, group 64, bf16, K = 4096 (before -> now):
+  // M = 1024 N = 11008 188 -> 162 us (572 TFLOP/s), M = 2048 N = 11008
+  // 369 -> 301, M = 1024 N = 32000 517 -> 429, M = 512 N = 11008 104 -> 86.
+  static constexpr bool QDMA = QB != 0 && BM == 128 && BN == 64;
+  // Scales and biases staged as fp32: no conversion in the computing waves
+  // (128 x 128, M = 1024 N = 11008: 196 -> 185 us). The smaller tiles lose by
+  // it (64 x 64: 188 -> 234 us, their registers pass 128 and a CU holds one
+  // workgroup instead of two).
+  static constexpr bool QF32 = QB != 0 && BM * BN >= 128 * 64;
+  static_assert(!QDMA || (QNT == NT && QLA == DMA_A), "every wave loads whole 1 KB blocks of A");
   static constexpr int GPS = EPS / 32;        // most groups that end in one stage
   static constexpr int QSB = BN * GPS;        // scale/bias entries staged per stage
   static constexpr int LSB = (QSB + QNT - 1) / QNT;
@@ -999,7 +1017,7 @@ struct GemmTile {
   // wave wait for every load in flight, the prefetched stages with them.
   using QWord = typename std::conditional<QB == 8, uint2, uint32_t>::type;
   struct QStage {
-    uint4 a[QLA];
+    uint4 a[QDMA ? 1 : QLA];          // (unused with QDMA)
     QWord w[LBU];                     // packed codes of unit i
     unsigned short sc[LSB], zb[LSB];  // scale and bias of entry i, element bits
   };
@@ -1027,6 +1045,10 @@ struct GemmTile {
     rz_src = make_rsrc(static_cast<const T*>(p.qz) + n0 * G, rows * G * E);
 #pragma unroll
     for (int i = 0; i < QLA; i++) {
+      if constexpr (QDMA) {
+        dma_addr(true, dma_blk(i), qa_off[i], qa_k[i]);
+        continue;
+      }
       const int q = qtid + i * QNT, r = q / RC, c = q % RC;
       qa_off[i] = (uint32_t)((r * K + c * EPC) * E);
       qa_k[i] = (A_CH % QNT == 0 || q < A_CH) ? c * EPC : INT32_MAX;
@@ -1042,6 +1064,8 @@ struct GemmTile {
       const int e = qtid + i * QNT, r = e / GPS, gi = e % GPS;
       qs_off[i] = (uint32_t)((r * G + gi) * E);
       qs_gi[i] = (QSB % QNT == 0 || e < QSB) ? gi : INT32_MAX;
+      // QDMA: no group past those of a stage (none would be in the last row).
+      if (QDMA && gi >= max(1, EPS >> qgshift)) qs_off[i] = kOutOfRange;
     }
   }
 
@@ -1049,14 +1073,59 @@ struct GemmTile {
   // powers of two, so one divides the other.
   __device__ __forceinline__ int64_t glo(int64_t s) const { return (s * EPS) >> qgshift; }
 
+  // QDMA kernels take whole stages only (K a multiple of EPS), so a load needs
+  // no bound on K: a stage's offset is scalar, the lanes' offsets stay as they
+  // are (rows past M or N start past the buffer's end), and stages past the
+  // last one read it again.
+  __device__ __forceinline__ int last_stage(int64_t s) const {
+    return min((int)s, (int)(K / EPS) - 1);
+  }
+  // Loads of a stage's codes, scales and biases (qload, with QDMA).
+  static constexpr int QNB = LBU + 2 * LSB;
+
+  // Issue this wave's LDS-DMA loads of stage s of A. Nothing that loads moves
+  // across: the wait before a stage's barrier counts the loads after these.
+  __device__ __forceinline__ void qdma(int64_t s, QSlot sl) const {
+    const int a_step = last_stage(s) * (int)(EPS * sizeof(T));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < QLA; i++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(ra_src, (lds_void_t*)(sl.a + dma_blk(i) * 64), 16,
+                                               qa_off[i], a_step, 0, 0);
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
   __device__ __forceinline__ void qload(int64_t s, QStage& st) const {
     constexpr uint32_t E = sizeof(T);
+    if constexpr (QDMA) {
+      static_assert(B_U % QNT == 0, "no unit index past a stage's last");
+      const int at = last_stage(s);
+      const int b_step = at * (EPS * QB / 8), s_step = (int)(glo(at) * E);
+#pragma unroll
+      for (int i = 0; i < LBU; i++) {
+        if constexpr (QB == 8)
+          st.w[i] = __builtin_bit_cast(
+              uint2, __builtin_amdgcn_raw_buffer_load_b64(rb_src, (int)qb_off[i], b_step, 0));
+        else
+          st.w[i] = __builtin_amdgcn_raw_buffer_load_b32(rb_src, (int)qb_off[i], b_step, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < LSB; i++) {
+        st.sc[i] = __builtin_amdgcn_raw_buffer_load_b16(rs_src, (int)qs_off[i], s_step, 0);
+        st.zb[i] = __builtin_amdgcn_raw_buffer_load_b16(rz_src, (int)qs_off[i], s_step, 0);
+      }
+      return;
+    }
     const int32_t kleft = (int32_t)(K - s * EPS);  // K elements from this stage on
     const uint32_t a_step = (uint32_t)(s * EPS) * E;
     const uint32_t b_step = (uint32_t)(s * EPS) * QB / 8;
+    if constexpr (!QDMA) {
 #pragma unroll
-    for (int i = 0; i < QLA; i++)
-      st.a[i] = buffer_chunk(ra_src, qa_k[i] < kleft ? qa_off[i] + a_step : kOutOfRange);
+      for (int i = 0; i < QLA; i++)
+        st.a[i] = buffer_chunk(ra_src, qa_k[i] < kleft ? qa_off[i] + a_step : kOutOfRange);
+    }
 #pragma unroll
     for (int i = 0; i < LBU; i++) {
       const uint32_t wo = qb_k[i] < kleft ? qb_off[i] + b_step : kOutOfRange;
@@ -1119,12 +1188,14 @@ struct GemmTile {
   // Stage st into LDS: A as loaded, B's codes as element-type integers in the
   // dense (N, K) tile layout, and the stage's scale/bias entries.
   __device__ __forceinline__ void qstore(QSlot sl, const QStage& st) const {
+    if constexpr (!QDMA) {
 #pragma unroll
-    for (int i = 0; i < QLA; i++) {
-      const int q = qtid + i * QNT;
-      if (A_CH % QNT == 0 || q < A_CH) {
-        const int r = q / RC, c = q % RC;
-        sl.a[r * RC + (c ^ swz_k<RC>(r))] = st.a[i];
+      for (int i = 0; i < QLA; i++) {
+        const int q = qtid + i * QNT;
+        if (A_CH % QNT == 0 || q < A_CH) {
+          const int r = q / RC, c = q % RC;
+          sl.a[r * RC + (c ^ swz_k<RC>(r))] = st.a[i];
+        }
       }
     }
 #pragma unroll
@@ -1154,8 +1225,12 @@ struct GemmTile {
     for (int i = 0; i < LSB; i++) {
       const int e = qtid + i * QNT;
       if (QSB % QNT == 0 || e < QSB) {
-        sl.s16[e] = st.sc[i];
-        sl.z16[e] = st.zb[i];
+        if constexpr (QF32) {
+          sl.sz[e % GPS * BN + e / GPS] = make_float2(bits_to_f32(st.sc[i]), bits_to_f32(st.zb[i]));
+        } else {
+          sl.s16[e] = st.sc[i];
+          sl.z16[e] = st.zb[i];
+        }
       }
     }
   }
@@ -1167,8 +1242,14 @@ struct GemmTile {
                                          f32x4_t (&P)[FM][FN], f32x4_t (&X)[FM]) const {
 #pragma unroll
     for (int jn = 0; jn < FN; jn++) {
-      const int at = (wn * WTN + jn * 16 + r16) * GPS + gi;
-      const float sc = bits_to_f32(sl.s16[at]), zb = bits_to_f32(sl.z16[at]);
+      const int col = wn * WTN + jn * 16 + r16;
+      float sc, zb;
+      if constexpr (QF32) {
+        const float2 sz = sl.sz[gi * BN + col];
+        sc = sz.x, zb = sz.y;
+      } else {
+        sc = bits_to_f32(sl.s16[col * GPS + gi]), zb = bits_to_f32(sl.z16[col * GPS + gi]);
+      }
 #pragma unroll
       for (int i = 0; i < FM; i++)
 #pragma unroll
@@ -1216,7 +1297,7 @@ struct GemmTile {
     constexpr int ng = GS <= EPS ? EPS / GS : 1;
     constexpr int per = (FN + 1) * FM * 4;  // registers of one group's P and X
     int cap = 1;
-    while (2 * cap * per <= 80) cap *= 2;
+    while (!QDMA && 2 * cap * per <= 80) cap *= 2;
     return ng < cap ? ng : cap;
   }
 
@@ -1230,11 +1311,13 @@ struct GemmTile {
                                                  f32x4_t (&P)[NGR][FM][FN],
                                                  f32x4_t (&X)[NGR][FM]) const {
     constexpr int CPG = GS / 32;  // chunk-steps per group
+    constexpr int AHEAD = QDMA ? 0 : 1;
     uint4 av[2][FM], bv[2][FN];
-    read_operands(Slot{sl.a, sl.b}, 0, av[0], bv[0]);
+    if constexpr (AHEAD) read_operands(Slot{sl.a, sl.b}, 0, av[0], bv[0]);
 #pragma unroll
     for (int j = 0; j < CS; j++) {
-      if (j + 1 < CS) read_operands(Slot{sl.a, sl.b}, j + 1, av[(j + 1) & 1], bv[(j + 1) & 1]);
+      if (j + AHEAD < CS)
+        read_operands(Slot{sl.a, sl.b}, j + AHEAD, av[(j + AHEAD) & 1], bv[(j + AHEAD) & 1]);
       if constexpr (GS <= EPS) {
         // Inside a stage a group starts at every CPG-th chunk-step.
         const int gi = j / CPG;
@@ -1293,9 +1376,11 @@ struct GemmTile {
     for (int64_t s0 = 0; s0 < nst; s0 += QP) {
 #pragma unroll
       for (int u = 0; u < QP; u++) {
-        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(63));
+        // QDMA: this stage's A has landed, the loads issued after it may not.
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm_lgkm0(QDMA ? QNB : 63));
         asm volatile("s_barrier" ::: "memory");
         if constexpr (LOAD) {
+          if constexpr (QDMA) qdma(s0 + u + 1, slots((u + 1) & 1));
           qstore(slots((u + 1) & 1), q[(u + 1) % QP]);
           qload(s0 + u + 1 + QP, q[(u + 1) % QP]);
         }
@@ -1335,6 +1420,7 @@ struct GemmTile {
       }
       return;
     }
+    if constexpr (QDMA) qdma(0, slots(0));
 #pragma unroll
     for (int u = 0; u < QP; u++) qload(u, q[u]);
     qstore(slots(0), q[0]);
@@ -1343,6 +1429,8 @@ struct GemmTile {
       q_rounds<true, true, GS, NGR>(slots, nst, nsteps, q, acc, P, X);
     else
       q_rounds<false, true, GS, NGR>(slots, nst, nsteps, q, acc, P, X);
+    // No load may still be landing in the LDS when the workgroup ends.
+    if constexpr (QDMA) __builtin_amdgcn_s_waitcnt(0);
   }
 
   // Register-staged path: stage s goes from registers to slot s mod 2 while
@@ -1585,15 +1673,18 @@ __global__ void __launch_bounds__(64 * NW) gemm_kernel(GemmArgs p) {
 // footprint only decides which elements a workgroup owns. One RNE rounding at
 // the end.
 template <typename T, int BM, int BN, int WM, int WN, int NW, int KB, int QB, int GS>
-__global__ void __launch_bounds__(64 * NW) gemm_qkernel(GemmArgs p) {
+__global__ void __launch_bounds__(64 * NW, (BM != 128 || BN != 64 ? 1 : GS == 64 ? 3 : 2) * NW / 4)
+gemm_qkernel(GemmArgs p) {
   using Tile = GemmTile<T, BM, BN, WM, WN, NW, KB, 2, true, QB>;
   constexpr int FM = Tile::FM, FN = Tile::FN;
   constexpr int AC = Tile::A_CH, BC = Tile::B_CH, SB = Tile::QSB;
   __shared__ uint4 a0[AC], b0[BC], a1[AC], b1[BC];
-  __shared__ unsigned short s0[SB], z0[SB], s1[SB], z1[SB];
+  constexpr int SB16 = Tile::QF32 ? 1 : SB, SB32 = Tile::QF32 ? SB : 1;
+  __shared__ unsigned short s0[SB16], z0[SB16], s1[SB16], z1[SB16];
+  __shared__ float2 f0[SB32], f1[SB32];
   auto slots = [&](int u) -> QSlot {
-    if (u == 0) return {a0, b0, s0, z0};
-    return {a1, b1, s1, z1};
+    if (u == 0) return {a0, b0, s0, z0, f0};
+    return {a1, b1, s1, z1, f1};
   };
 
   Tile t;
@@ -1666,7 +1757,8 @@ __global__ void __launch_bounds__(64 * NW) gemm_qkernel(GemmArgs p) {
   X(4, 256, 128, 4, 2, 12, 128, 3, 1, 0)     \
   X(5, 64, 32, 4, 2, 8, 256, 3, 0, 0)        \
   X(6, 256, 256, 4, 4, 16, 64, 4, 0, 1)      \
-  X(7, 256, 256, 2, 2, 4, 128, 5, 0, 2)
+  X(7, 256, 256, 2, 2, 4, 128, 5, 0, 2)      \
+  X(8, 128, 64, 4, 1, 4, 128, 3, 0, 0)
 
 using KernelFn = void (*)(GemmArgs);
 
@@ -1680,7 +1772,8 @@ namespace bi_gemm_dev {
 // Kernel for geometry g in the translation unit of element type T; ragged:
 // its register-staged form for operands that are not 16-byte aligned (the
 // footprints with loading waves or more than 8 waves have none: the staged
-// loads' registers would make them spill).
+// loads' registers would make them spill; nor has 128 x 64, which is there for
+// many rows of aligned and quantized operands).
 template <typename T>
 KernelFn kernel_for(int g, bool trans_b, bool ragged) {
 // fp32 carries two accumulator chains per element: with more than 8 waves
@@ -1688,7 +1781,7 @@ KernelFn kernel_for(int g, bool trans_b, bool ragged) {
 #define BI_GEO_CASE(id, bm, bn, wm, wn, nw, kb, ns, pl, pp)                             \
   case id:                                                                             \
     if (ragged) {                                                                      \
-      if constexpr (!pl && !pp)                                                        \
+      if constexpr (!pl && !pp && !(bm == 128 && bn == 64))                            \
         return trans_b ? gemm_kernel<T, bm, bn, wm, wn, nw, kb, 2, true, 0, 0, true>   \
                        : gemm_kernel<T, bm, bn, wm, wn, nw, kb, 2, false, 0, 0, true>; \
       return nullptr;                                                                  \

@@ -130,6 +130,43 @@ def test_every_geometry_gives_the_same_bits(cuda):
 
 
 @pytest.mark.parametrize("dname,dtype", QDTYPES)
+@pytest.mark.parametrize("gs", [32, 64, 128])
+def test_prefill_footprint_gives_the_same_bits(cuda, dname, dtype, gs):
+    """The prefill footprint (128 x 64, the activations straight into LDS, whole
+    stages of K only) gives the 16x16 footprint's bits: one stage and many,
+    rows and columns cut short, several tiles, an infinity and a NaN in the
+    activations. K that is no multiple of a stage, or 0, is refused."""
+    L = _lib.lib()
+    pre = bi.geometries().index((128, 64, 4))
+    assert L.bi_qgemm_pick_geometry(1024, 11008, 4096, 4) == pre
+    assert L.bi_qgemm_pick_geometry(1024, 11008, 4096 + 32, 4) != pre
+    for nbits in (2, 4, 8):
+        for M, N, K in [(1, 1, 128), (128, 64, 128), (129, 65, 384), (300, 130, 2048),
+                        (127, 200, 640), (513, 16, 4096)]:
+            q, s, b = _qweight(N, K, dtype, 160 + gs + M + nbits, gs, nbits, cuda)
+            x = rn((M, K), dtype, 161 + K, device=cuda)
+            if M > 1:
+                x[M // 2, K // 3] = float("inf")
+                x[M - 1, K - 1] = float("nan")
+            want = bits(_launch(L, x, q, s, b, gs, nbits, 0))
+            got = bits(_launch(L, x, q, s, b, gs, nbits, pre))
+            assert np.array_equal(got, want), (nbits, M, N, K)
+    if gs < 128:
+        for K in (64, 192):  # one stage; an odd number of stages
+            q, s, b = _qweight(70, K, dtype, 163, gs, 4, cuda)
+            x = rn((130, K), dtype, 164, device=cuda)
+            assert np.array_equal(bits(_launch(L, x, q, s, b, gs, 4, 0)),
+                                  bits(_launch(L, x, q, s, b, gs, 4, pre)))
+    if gs == 32:
+        q, s, b = _qweight(64, 96, dtype, 165, gs, 4, cuda)
+        with pytest.raises(NotImplementedError):
+            _launch(L, rn((128, 96), dtype, 166, device=cuda), q, s, b, gs, 4, pre)
+    with pytest.raises(NotImplementedError):
+        _launch(L, x[:, :0].contiguous(), q[:, :0].contiguous(), s[:, :0].contiguous(),
+                b[:, :0].contiguous(), gs, 4, pre)
+
+
+@pytest.mark.parametrize("dname,dtype", QDTYPES)
 def test_decode_footprint_gives_the_same_bits(cuda, dname, dtype):
     """The decode footprint (2-, 4- and 8-bit weights, at most 8 rows: the waves of
     a workgroup split K by groups, the codes reach the matrix cores through a
