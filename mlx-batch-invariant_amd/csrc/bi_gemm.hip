@@ -92,7 +92,10 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
   if (M <= 128) {
     // 65..128 rows: 128 x 128 tiles on wide weights (a 256-row tile would be
     // mostly padding), 64 x 32 on narrow ones.
-    if (t128 >= 80) return 3;
+    // A (K, N) weight whose 64-column tiles fit one round takes 128 x 64: twice
+    // the workgroups stream it (M = 100, N = 11008, K = 4096: 25.1 us against
+    // 30.5; with an (N, K) weight both 25).
+    if (t128 >= 80) return !trans_b && ceil_div(N, 64) <= 256 ? 8 : 3;
     return t64 >= 192 ? 2 : 5;
   }
   if (M <= 256) {
@@ -112,11 +115,15 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
   // 128 of them, 92 us against 63 us for 256 x 128). On (N, K) weights the
   // four-wave 256 x 256 footprint takes its place: equal or faster on every
   // measured cell (M = 512..4096, N = 4096..32000, K = 4096..14336; M = 4096,
-  // K = 11008, N = 4096: 260 against 298 us), 7 % faster on average.
+  // K = 11008, N = 4096: 260 against 298 us), 7 % faster on average. 128 x 64
+  // tiles are the ones where they fit one round and 64 x 64 ones take two (K =
+  // 11008, N = 4096, M = 300: 56.9 against 67.1 us, (K, N) 61.0 against 68.1;
+  // N = K = 2048, M = 1024: 13.5 against 15.6).
   struct Cand { int g, bm, bn, w; };
   const Cand kCands[] = {{2, 64, 64, 129},
                          {3, 128, 128, 136},
                          {4, 256, 128, 144},
+                         {8, 128, 64, 158},
                          trans_b ? Cand{7, 256, 256, 180} : Cand{6, 256, 256, 192}};
   int best = 2;
   int64_t best_cost = -1;
