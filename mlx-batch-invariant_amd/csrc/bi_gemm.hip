@@ -142,8 +142,8 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
 // for 17..64 rows of a narrow weight; 64 x 64 for 17..64 rows of a wide one
 // (N = 32000, M = 32: 37 us against 86 us for 64 x 16); above that the
 // dense rules, except that 128 x 128 must fill the CUs (its workgroups
-// dequantize twice the columns: N = 11008, M = 256: 64 x 64 61 us, 128 x 128
-// 70 us).
+// dequantize twice the columns: N = 11008, M = 256: 64 x 64 58 us, 128 x 128
+// 63 us), and more than 256 rows have a rule of their own.
 // Id of the quantized decode footprint (bi_gemm_qdecode.h: 2-, 4- or 8-bit
 // codes, at most 8 rows), one past the dense table.
 constexpr int kQDecode = kNumGeometries;
