@@ -23,7 +23,7 @@ __device__ __forceinline__ FoldW fold_stats(float& R, float& S, float M, float L
 }
 __device__ __forceinline__ void fold_out(f32x4_t& Q, const f32x4_t& O, FoldW w) {
 #pragma unroll
-  for (int e = 0; e < 4; e++) Q[e] = __builtin_fmaf(O[e], w.f, __builtin_fmaf(Q[e], w.e, 0.f));
+  for (int e = 0; e < 4; e++) Q[e] = __builtin_fmaf(O[e], w.f, Q[e] * w.e) + 0.f;
 }
 
 }  // namespace

@@ -49,9 +49,12 @@
 //     simdgroup 0, would put a large sink's p below f16's range.)
 //   * The segments fold in ascending order: the first segment's (M, L, O) is
 //     the running (R, S, Q); then R' = max(R, M), e = exp2(R - R'),
-//     f = exp2(M - R'), S = fma(L, f, S * e), Q = fma(O, f, fma(Q, e, 0))
-//     (never -0.0, so a segment without a usable key changes no bit).
-//     out = S == 0 ? Q : Q / S, one rounding to T.
+//     f = exp2(M - R'), S = fma(L, f, S * e), Q = fma(O, f, Q * e) + 0.0.
+//     out = S == 0 ? Q : Q / S, one rounding to T, of Q + 0.0 where there is
+//     one segment: a product that underflows from below leaves -0.0, which
+//     the addition turns into +0.0, so Q is never -0.0, a segment without a
+//     usable key (f == 0 or O == 0) changes no bit of it, and neither does
+//     the number of such segments or which of them a launch skips.
 //     Segments lie at fixed keys, so whether one workgroup walks them all or
 //     each has its own workgroup changes nothing a column computes.
 // Every column, whatever workgroup or lane it lands in, however many rows or
@@ -1084,6 +1087,8 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
         if constexpr (SEG == SEG_WALK) {
           fold_out(r.Q[k], O, w);
           O = r.Q[k];
+        } else {
+          O += 0.f;
         }
         unsigned short ob[4];
 #pragma unroll
@@ -1564,6 +1569,8 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
       if (folded) Q = __builtin_bit_cast(f32x4_t, ld16(run_lds() + (wave * NB + db) * 64 + lane));
       fold_out(Q, O, w);
       O = Q;
+    } else {
+      O += 0.f;
     }
     unsigned short ob[4];
 #pragma unroll

@@ -533,3 +533,57 @@ def test_segments_give_the_same_bits_in_one_workgroup_or_each_in_its_own(cuda, D
             # 2^-9 bf16, 2^-12 f16, per product of the sum): 2-norm within 2.5 of it.
             err = np.linalg.norm(f64(base) - want) / np.linalg.norm(want)
             assert err < 2.5 * 2.0 ** (-9 if dname == "bfloat16" else -12), (dname, N, mode, err)
+
+
+def _underflowing(B, H, Hkv, qL, N, D, dtype, device, low_block, rest):
+    """A problem whose output is a negative product below the fp32 range: key 0
+    scores 120 (base 2) above the first key of block `low_block`, and that one
+    10 above the second, whose values are -2^-24; all other values are 0 and
+    the other keys score `rest`. Every output is -2^-154."""
+    q = torch.zeros(B, H, qL, D, dtype=dtype, device=device)
+    k = torch.zeros(B, Hkv, N, D, dtype=dtype, device=device)
+    v = torch.zeros(B, Hkv, N, D, dtype=dtype, device=device)
+    ln2 = math.log(2.0)
+    j = 32 * low_block
+    q[..., 0] = 1.0
+    k[..., 0] = rest * ln2
+    k[:, :, 0, 0] = 120 * ln2
+    k[:, :, j, 0] = 0
+    k[:, :, j + 1, 0] = -10 * ln2
+    v[:, :, j + 1] = -2.0 ** -24
+    keep = torch.zeros(1, 1, 1, N, dtype=torch.bool, device=device)
+    keep[..., [0, j, j + 1]] = True
+    return q, k, v, keep
+
+
+@pytest.mark.parametrize("dname,dtype", LOW)
+def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
+    """A negative result below the fp32 range is +0.0 in every launch shape,
+    with one segment of keys or with more behind it (hidden by the mask, or by
+    the causal bound), walked or one per workgroup: its sign does not depend
+    on the context's length or on the route."""
+    B, H, Hkv, qL, D = 1, 8, 2, 5, 128
+    for low_block in (3, 2, 67):  # the last chain, an earlier one, the second segment
+        for N in (2048, 2112, 4300, 8192):
+            if 32 * low_block >= N:
+                continue
+            q, k, v, keep = _underflowing(B, H, Hkv, qL, N, D, dtype, cuda, low_block, 0)
+            for split in (False, True):
+                for shape in range(_lib.SDPA_NUM_SHAPES):
+                    if shape == _lib.SDPA_SHARED:
+                        continue  # no array mask
+                    mode, m, ms, off = _mask_mode(keep, q, k)
+                    y = _attention._sdpa_eager(q, k, v, 1.0, mode, m, ms, off, None, shape=shape,
+                                               split=split)
+                    assert not bits(y).any(), (dname, low_block, N, shape, split)
+    # Without a mask: the other keys score far below both (by 400), causal rows
+    # of the shared shape among them.
+    for N in (2048, 4300):
+        q, k, v, _ = _underflowing(B, H, Hkv, 64, N, D, dtype, cuda, 3, -400)
+        for spec in (None, "start"):
+            for shape in range(_lib.SDPA_NUM_SHAPES):
+                mode, m, ms, off = _mask_mode(spec, q, k)
+                if spec:
+                    off = 2000  # rows 0..63 see keys up to 2000..2063
+                y = _attention._sdpa_eager(q, k, v, 1.0, mode, m, ms, off, None, shape=shape)
+                assert not bits(y).any(), (dname, N, spec, shape)
