@@ -143,7 +143,12 @@ def _launch(L, args, shape, split, q, stream):
         return L.bi_sdpa(*args, stream)
     # Used by this stream's launches only, so the caching allocator may give
     # it to the next call on the stream as soon as it is dropped here.
-    ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+    try:
+        ws = torch.empty(need, dtype=torch.uint8, device=q.device)
+    except torch.OutOfMemoryError:
+        if split:
+            raise
+        return L.bi_sdpa(*args, stream)  # the same bits without a workspace
     if split:
         return L.bi_sdpa_split_with_shape(*args, int(shape), ws.data_ptr(), need, stream)
     return L.bi_sdpa_ws(*args, ws.data_ptr(), need, stream)

@@ -576,3 +576,32 @@ def test_quantized_linear_validation():
     # outside the mode quantized_matmul is stock: dequantize, then F.linear
     y = bi.quantized_matmul(x, w, s, b, True, 64, 4)
     assert torch.equal(y, F.linear(x, bi.dequantize(w, s, b, 64, 4)))
+
+
+def test_attention_runs_without_a_workspace_it_cannot_get(monkeypatch):
+    """bi_sdpa gives the same bits as bi_sdpa_ws without a workspace: a call
+    whose workspace cannot be allocated takes it instead of failing."""
+    class Recording:
+        calls = []
+
+        def bi_sdpa_workspace(self, *args):
+            return 1 << 20
+
+        def bi_sdpa(self, *args):
+            self.calls.append("bi_sdpa")
+            return _lib.OK
+
+        def bi_sdpa_ws(self, *args):
+            self.calls.append("bi_sdpa_ws")
+            return _lib.OK
+
+    L, q = Recording(), torch.zeros(1, 8, 1, 128, dtype=torch.bfloat16)
+    args = (0, 0, 0, None, None, None, 0, 1, 8, 2, 1, 8192, 128, 128, None, 1.0, 0, 8191, _lib.BF16)
+    assert _attention._launch(L, args, None, False, q, 0) == _lib.OK
+
+    def full(*args, **kwargs):
+        raise torch.OutOfMemoryError("out of memory")
+
+    monkeypatch.setattr(torch, "empty", full)
+    assert _attention._launch(L, args, None, False, q, 0) == _lib.OK
+    assert L.calls == ["bi_sdpa_ws", "bi_sdpa"]
