@@ -173,7 +173,9 @@ int pick_qgeometry(int64_t M, int64_t N, int64_t K, int bits, int group) {
     if (t128 >= 160) return 3;
     return t64 >= 192 ? 2 : 5;
   }
-  if (M <= 256 || K % kQPrefillStage)
+  // (128 rows of 2^23 or more activations pass the 2 GiB of a buffer resource;
+  // the 64 of a 64 x 64 tile may still fit.)
+  if (M <= 256 || K % kQPrefillStage || K >= (int64_t)1 << 23)
     return (M <= 256 ? t128 : ceil_div(N, 128)) >= 200 ? 3 : 2;
   // More rows: 64 x 64 tiles or the prefill footprint's 128 x 64, whichever
   // has the less estimated time: rounds of 256 workgroups times a round's

@@ -125,6 +125,17 @@ def test_quantized_footprint_policy():
     assert L.bi_qgemm_pick_geometry(1, 4096, 4096, 3) == _lib.EINVAL
 
 
+def test_wide_tiles_are_not_picked_past_their_panel_limit():
+    """A tile's rows of A must fit a 2 GiB buffer resource: K = 2^23 16-bit
+    elements pass it in 128 rows and not in 64, so more than 256 rows keep the
+    64 x 64 footprint there."""
+    L = _lib.lib()
+    geos = bi.geometries()
+    quant = lambda K: geos[L.bi_qgemm_pick_geometry(1024, 11008, K, 4)]
+    assert quant((1 << 23) - 64) == (128, 64, 4)
+    assert quant(1 << 23) == (64, 64, 8)
+
+
 def _err():
     return _lib.lib().bi_last_error().decode()
 
