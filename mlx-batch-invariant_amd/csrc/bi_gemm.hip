@@ -65,7 +65,7 @@ int pick_geometry_f32(int64_t M, int64_t N) {
   return 2;
 }
 
-int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
+int pick_geometry(int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
   const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);  // 128 x 128 tiles
   const int64_t t64 = ceil_div(M, 64) * ceil_div(N, 64);     // 64 x 64 tiles
   // Decode: 16 x 16 tiles in a 64 KB ring, two workgroups per CU, so one
@@ -118,7 +118,9 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
   // K = 11008, N = 4096: 260 against 298 us), 7 % faster on average. 128 x 64
   // tiles are the ones where they fit one round and 64 x 64 ones take two (K =
   // 11008, N = 4096, M = 300: 56.9 against 67.1 us, (K, N) 61.0 against 68.1;
-  // N = K = 2048, M = 1024: 13.5 against 15.6).
+  // N = K = 2048, M = 1024: 13.5 against 15.6) and their 128 rows of A fit a
+  // buffer resource.
+  const bool panel = K < (int64_t)1 << 23;
   struct Cand { int g, bm, bn, w; };
   const Cand kCands[] = {{2, 64, 64, 129},
                          {3, 128, 128, 136},
@@ -128,6 +130,7 @@ int pick_geometry(int64_t M, int64_t N, int dtype, int trans_b) {
   int best = 2;
   int64_t best_cost = -1;
   for (const Cand& c : kCands) {
+    if (c.g == 8 && !panel) continue;
     const int64_t cost = ceil_div(ceil_div(M, c.bm) * ceil_div(N, c.bn), 256) * (c.bm + c.bn) * c.w;
     if (best_cost < 0 || cost < best_cost) {
       best = c.g;
@@ -277,7 +280,7 @@ int pick_ragged(int64_t M, int64_t N, int dtype, int trans_b) {
 // The geometry bi_gemm launches: pick_geometry's for operands whose every
 // row may be read as aligned 16-byte vectors by it, else pick_ragged's.
 int pick_for(const void* a, const void* b, int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
-  const int g = pick_geometry(M, N, dtype, trans_b);
+  const int g = pick_geometry(M, N, K, dtype, trans_b);
   const VecFlags v = vec_flags(a, b, N, K, dtype, trans_b, kGeometries[g]);
   return v.a && v.b ? g : pick_ragged(M, N, dtype, trans_b);
 }
@@ -413,8 +416,7 @@ extern "C" int bi_gemm_geometry_info(int g, int* block_m, int* block_n, int* wav
 }
 
 extern "C" int bi_gemm_pick_geometry(int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
-  (void)K;
-  return pick_geometry(M, N, dtype, trans_b);
+  return pick_geometry(M, N, K, dtype, trans_b);
 }
 
 extern "C" int bi_gemm_with_geometry(const void* a, const void* b, const void* bias, void* out,

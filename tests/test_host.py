@@ -131,6 +131,9 @@ def test_wide_tiles_are_not_picked_past_their_panel_limit():
     64 x 64 footprint there."""
     L = _lib.lib()
     geos = bi.geometries()
+    dense = lambda K: geos[L.bi_gemm_pick_geometry(300, 4096, K, _lib.BF16, 1)]
+    assert dense((1 << 23) - 8) == (128, 64, 4)
+    assert dense(1 << 23) == (64, 64, 8)
     quant = lambda K: geos[L.bi_qgemm_pick_geometry(1024, 11008, K, 4)]
     assert quant((1 << 23) - 64) == (128, 64, 4)
     assert quant(1 << 23) == (64, 64, 8)
