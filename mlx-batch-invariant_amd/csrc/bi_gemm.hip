@@ -559,10 +559,17 @@ extern "C" int bi_qgemm(const void* x, const void* w, const void* scales, const 
 
 extern "C" int bi_qgemm_num_geometries(void) { return kQDecode + 1; }
 
-extern "C" int bi_qgemm_pick_geometry(int64_t M, int64_t N, int64_t K, int bits) {
+extern "C" int bi_qgemm_pick_group_geometry(int64_t M, int64_t N, int64_t K, int group_size,
+                                            int bits) {
   if (bits != 2 && bits != 4 && bits != 8)
     return bi::fail(BI_EINVAL, "bi_qgemm: bits must be 2, 4 or 8, got %d", bits);
-  return pick_qgeometry(M, N, K, bits, 64);
+  if (group_shift(group_size) < 0)
+    return bi::fail(BI_EINVAL, "bi_qgemm: group size must be 32, 64 or 128, got %d", group_size);
+  return pick_qgeometry(M, N, K, bits, group_size);
+}
+
+extern "C" int bi_qgemm_pick_geometry(int64_t M, int64_t N, int64_t K, int bits) {
+  return bi_qgemm_pick_group_geometry(M, N, K, 64, bits);
 }
 
 extern "C" int bi_qgemm_with_geometry(const void* x, const void* w, const void* scales,

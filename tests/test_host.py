@@ -125,6 +125,25 @@ def test_quantized_footprint_policy():
     assert L.bi_qgemm_pick_geometry(1, 4096, 4096, 3) == _lib.EINVAL
 
 
+def test_quantized_footprint_by_group_size():
+    """More than 256 rows: 64 x 64 or 128 x 64 tiles by rounds of workgroups
+    whose times depend on the group size (M = 1024, N = 11008: 128 x 64 for
+    groups of 32 and 64 only). bi_qgemm_pick_geometry answers for 64."""
+    L = _lib.lib()
+    geos = bi.geometries()
+    pick = lambda M, N, gs, bits=4: geos[L.bi_qgemm_pick_group_geometry(M, N, 4096, gs, bits)]
+    small, large = (64, 64, 8), (128, 64, 4)
+    assert [pick(1024, 11008, gs) for gs in (32, 64, 128)] == [large, large, small]
+    assert [pick(512, 4096, gs) for gs in (32, 64, 128)] == [small, small, small]
+    assert [pick(1024, 32000, gs) for gs in (32, 64, 128)] == [large, large, large]
+    for bits in (2, 4, 8):
+        for M in (1, 8, 40, 100, 256, 300, 1024):
+            assert (L.bi_qgemm_pick_geometry(M, 11008, 4096, bits)
+                    == L.bi_qgemm_pick_group_geometry(M, 11008, 4096, 64, bits))
+    assert L.bi_qgemm_pick_group_geometry(1, 4096, 4096, 64, 3) == _lib.EINVAL
+    assert L.bi_qgemm_pick_group_geometry(1, 4096, 4096, 48, 4) == _lib.EINVAL
+
+
 def test_wide_tiles_are_not_picked_past_their_panel_limit():
     """A tile's rows of A must fit a 2 GiB buffer resource: K = 2^23 16-bit
     elements pass it in 128 rows and not in 64, so more than 256 rows keep the
