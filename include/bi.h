@@ -97,14 +97,13 @@ int bi_gemm(const void* a, const void* b, const void* bias, void* out,
  *
  * One fixed reduction per element type. BI_F32: key i is owned by partial
  * (i mod 32) and walked in ascending order; the 32 partials are combined in a
- * fixed order. BI_F16 / BI_BF16 (matrix cores): keys are taken in segments of
- * 2048 and blocks of 32, block b owned by chain (b mod 4) of its segment and
- * walked in ascending order; the 4 chains are combined in a fixed order, and
- * the segments' results folded in ascending order. Nothing in the reduction depends on
+ * fixed order. BI_F16 / BI_BF16 (matrix cores): keys are taken in blocks of
+ * 32, block b owned by chain (b mod 4) and walked in ascending order; the 4
+ * chains are combined in a fixed order. Nothing in the reduction depends on
  * B, qL, the other query rows, or N beyond which keys exist, so growing the
  * context with masked keys leaves earlier results bitwise unchanged. A query
  * row whose keys are all masked yields 0. A sink enters the fixed-order
- * combine of the first segment as one more partial (m = sink, l = 1, o = 0).
+ * combine as one more partial (m = sink, l = 1, o = 0).
  * Keys that no query row can see -- past every row's causal bound (e.g. an
  * unwritten cache tail) or hidden by an array mask from every query sharing a
  * workgroup -- never reach the output, whatever they hold (the reference skips
@@ -131,9 +130,9 @@ int bi_sdpa(const void* q, const void* k, const void* v,
             int dtype, void* hip_stream);
 
 /*
- * Bytes of device memory with which bi_sdpa_ws runs this problem over more
- * workgroups than bi_sdpa (one per segment of the keys); 0 if it would not.
- * The current device's compute units decide.
+ * Bytes of device memory with which bi_sdpa_ws is expected to run this problem
+ * faster than bi_sdpa; 0 if it would not use any. The current device's compute
+ * units decide, and at most 256 MiB are asked for.
  */
 int64_t bi_sdpa_workspace(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N,
                           int64_t D, int64_t V, int dtype, int mask_mode);
@@ -141,8 +140,10 @@ int64_t bi_sdpa_workspace(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t
 /*
  * bi_sdpa, the same bits, with `workspace_bytes` bytes of device memory (at
  * least bi_sdpa_workspace's, 16-byte aligned; with less, or NULL, it is
- * bi_sdpa). The call overwrites the memory; it must stay allocated, and
- * unused by others, until the call's work on the stream has run.
+ * bi_sdpa). A first kernel then writes the raw scores there, its workgroups
+ * sharing out the keys, and bi_sdpa's reduction reads them. The call overwrites
+ * the memory; it must stay allocated, and unused by others, until the call's
+ * work on the stream has run.
  */
 int bi_sdpa_ws(const void* q, const void* k, const void* v,
                const void* mask, const int64_t* mask_strides,

@@ -121,8 +121,10 @@ int bi_sdpa_with_shape(const void* q, const void* k, const void* v,
                        float scale, int mask_mode, int64_t causal_offset,
                        int dtype, int shape, void* hip_stream);
 
-/* bi_sdpa_ws with one segment of the keys per workgroup, in launch shape
- * `shape` (BI_F16 / BI_BF16; any but "shared"), whatever the size. */
+/* bi_sdpa_ws with the scores by a kernel of their own, read in launch shape
+ * `shape` (BI_F16 / BI_BF16; any but "shared", "rows" as "tile"), whatever the
+ * size. The workspace takes B * Hkv * ceil(c / 16) * ceil(N / 32) blocks of
+ * 128 * min(c, 16) bytes, c = H / Hkv * qL. */
 int bi_sdpa_split_with_shape(const void* q, const void* k, const void* v,
                              const void* mask, const int64_t* mask_strides,
                              const void* sinks, void* out,

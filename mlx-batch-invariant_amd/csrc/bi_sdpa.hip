@@ -7,9 +7,10 @@
 // row of a few heads (the query heads of one kv head that share its keys
 // under grouped-query attention); keys are split over a fixed number of
 // partial online softmaxes by key index; the partials are combined in a fixed
-// order. There is no split-KV, no second pass and no route switch on query
-// length or context length. How many heads share a workgroup changes only
-// which loads are shared, never a head's arithmetic.
+// order. There is no split-KV. How many heads share a workgroup changes only
+// which loads are shared, never a head's arithmetic; so does, for bf16 and f16,
+// whether a workgroup computes its raw scores or reads those of a kernel that
+// ran before it (SdpaStage).
 //
 // Fixed per-row arithmetic (the invariance contract):
 //   * 256 threads = 4 waves x 8 groups of 8 lanes = 32 partials. Key i belongs
@@ -32,7 +33,6 @@
 //     out = L == 0 ? o : o / L (reference :124-141), one rounding to T.
 #include <hip/hip_runtime.h>
 #include <float.h>
-#include <math.h>
 #include <atomic>
 #include <stdint.h>
 
@@ -40,7 +40,6 @@
 
 #include "bi_internal.h"
 #include "bi_sdpa_args.h"
-#include "bi_sdpa_fold.h"
 
 namespace {
 
@@ -48,6 +47,7 @@ constexpr int kThreads = 256;
 constexpr int64_t kMaskSlack = 64;  // keys a block may read past N
 constexpr int kPartials = 32;
 constexpr int kGroupLanes = 8;
+constexpr float kLog2e = 1.4426950408889634f;
 
 template <typename T> __device__ inline float to_f32(T x) { return (float)x; }
 // A mask element held as its zero-extended bits (16-bit types) or as itself
@@ -369,47 +369,10 @@ SdpaKernelFn f32_kernel(int64_t D, int64_t V, int shape) {
 
 // ---------------------------------------------------------------- MFMA shapes
 
-// Folds the segments' partial results (SdpaArgs::part) in ascending order and
-// writes the output; one thread per column and 4 dims. Bound by the launch and
-// one round of loads, eight segments at a time (about 2.5 us in all).
-template <typename T>
-__global__ void __launch_bounds__(256) sdpa_fold_kernel(SdpaArgs p, int V) {
-  const int quads = V / 4;
-  const int64_t ncol = p.B * p.H * p.qL;
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t col = i / quads;
-  if (col >= ncol) return;
-  const int d = (int)(i % quads) * 4;
-  const float* __restrict__ po = p.part + col * p.nseg * V + d;
-  const float2* __restrict__ pm =
-      reinterpret_cast<const float2*>(p.part + ncol * p.nseg * V) + col * p.nseg;
-  // (The fold of the first segment into this state leaves it as it is.)
-  float R = -FLT_MAX, S = 0.f;
-  f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  constexpr int A = 8;
-  for (int s0 = 0; s0 < p.nseg; s0 += A) {
-    f32x4_t O[A];
-    float2 st[A];
-#pragma unroll
-    for (int u = 0; u < A; u++) {
-      const int s = s0 + u < p.nseg ? s0 + u : p.nseg - 1;
-      O[u] = *reinterpret_cast<const f32x4_t*>(po + (int64_t)s * V);
-      st[u] = pm[s];
-    }
-#pragma unroll
-    for (int u = 0; u < A; u++)
-      if (s0 + u < p.nseg) fold_out(Q, O[u], fold_stats(R, S, st[u].x, st[u].y));
-  }
-  unsigned short ob[4];
-#pragma unroll
-  for (int e = 0; e < 4; e++) ob[e] = __builtin_bit_cast(unsigned short, (T)(S == 0.f ? Q[e] : Q[e] / S));
-  *reinterpret_cast<uint2*>(static_cast<T*>(p.out) + col * V + d) =
-      make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
-}
-
-SdpaKernelFn mfma_kernel(int64_t D, int64_t V, int dtype, bool mask, int shape, int seg) {
+SdpaKernelFn mfma_kernel(int64_t D, int64_t V, int dtype, bool mask, int shape,
+                         int stage = SDPA_WHOLE) {
 #define BI_MFMA_CASE(d, v) \
-  if (D == d && V == v) return sdpa_mfma_kernel_d##d##_v##v(dtype, mask, shape, seg);
+  if (D == d && V == v) return sdpa_mfma_kernel_d##d##_v##v(dtype, mask, shape, stage);
   BI_SDPA_DIM_PAIRS(BI_MFMA_CASE)
 #undef BI_MFMA_CASE
   return nullptr;
@@ -484,86 +447,89 @@ bool shape_geometry(int64_t D, int64_t V, int dtype, int shape, int* columns, in
     *splits = 1;
     return true;
   }
-  if (shape < 0 || shape >= SDPA_NUM_SHAPES || !mfma_kernel(D, V, dtype, false, shape, SEG_ONE))
+  if (shape < 0 || shape >= SDPA_NUM_SHAPES || !mfma_kernel(D, V, dtype, false, shape))
     return false;
   *columns = sdpa_shape_columns(D, V, shape);
   *splits = sdpa_shape_splits(V, shape);
   return true;
 }
 
-int64_t segments(int64_t N) { return N > 0 ? (N + kSegKeys - 1) / kSegKeys : 1; }
-
-// Bytes of partial results (SdpaArgs::part) of a launch over segments.
-int64_t split_bytes(int64_t B, int64_t H, int64_t qL, int64_t N, int64_t V) {
-  return B * H * qL * segments(N) * (V + 2) * (int64_t)sizeof(float);
+// The scores route (SdpaStage): raw scores by a kernel of their own, whose
+// workgroups share out the keys, then the rest of each column from memory.
+struct Scores {
+  int nsc, scw, bpw, tiles;  // SdpaArgs; column tiles per workgroup of the scores kernel
+  int64_t bytes, blocks;     // of the scores; workgroups of the scores kernel
+};
+Scores scores_plan(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int cus) {
+  Scores r;
+  const int64_t ncol = H / Hkv * qL, ncb = (ncol + 15) / 16, nsc = (N + 31) / 32;
+  r.nsc = (int)nsc;
+  r.scw = ncol < 16 ? (int)ncol : 16;
+  r.tiles = sdpa_score_tiles(D, ncol);
+  r.bytes = B * Hkv * ncb * nsc * 32 * r.scw * (int64_t)sizeof(float);
+  // Two workgroups of four waves per CU, each wave at least one block.
+  const int64_t groups = B * Hkv * ((ncb + r.tiles - 1) / r.tiles);
+  const int64_t bpw = (groups * nsc + 8 * cus - 1) / (8 * cus);
+  r.bpw = (int)(bpw < 1 ? 1 : bpw > 16 ? 16 : bpw);
+  r.blocks = groups * ((nsc + 4 * r.bpw - 1) / (4 * r.bpw));
+  return r;
 }
 
-// Estimated microseconds of a matrix-core launch whose workgroups each walk
-// `keys` of a segment's (or, nseg 1, of the whole context's) keys: the longest
-// of a chain's own time for its blocks, the key and value bytes that leave
-// HBM once per stream, and those that reach the workgroups through the L2s,
-// plus 4.5 for the launch's fixed parts. Fitted to a grid of B = 1..64, N =
-// 2100..8192, 1..32 query rows, D = 64, 128, 256, with and without an array
-// mask; a loader-wave workgroup fills a CU, so a few of them past a multiple
-// of the CUs cost a round.
-float estimate(int64_t D, int64_t V, int64_t tiles, int64_t streams, int shape, bool array_mask,
-               int64_t nseg, float keys, float walk, int cus) {
-  const bool loaders = sdpa_loaders(D, V, shape, array_mask);
-  const bool rows = shape == SDPA_ROWS && sdpa_rows_tiles(D, V) == 2;
-  const int ws = sdpa_shape_splits(V, shape);
-  const float dv = (float)(D + V), inv = 1.f / (float)ws;
-  const float chain = loaders ? 10.6f + 0.4f * inv                    // per 2048 keys
-                      : rows  ? 0.09f * dv
-                              : 6.f + (0.045f + 0.012f * inv) * dv;
-  float wgs = (float)((rows ? (tiles + streams) / 2 : tiles) * ws * nseg) / (float)cus;
-  if (loaders && wgs > 1.f) wgs = ceilf(wgs);
-  float hbm = 0.184f * dv * (float)(streams * nseg) / (float)cus;
-  if (ws == 1 && wgs < 1.f) hbm *= 1.15f;
-  if (nseg > 1) hbm *= 1.08f;
-  const float l2 = (rows ? (array_mask ? 0.15f : 0.105f) * dv
-                         : (nseg > 1 ? 0.132f : ws == 1 ? 0.09f : ws == 2 ? 0.075f : 0.098f) *
-                               ((float)D + (float)V * inv)) * wgs;
-  const float a = chain * walk / 2048.f, b = (hbm > l2 ? hbm : l2) * keys / 2048.f;
-  return 4.5f + (a > b ? a : b);
+// Whether a problem's offsets fit the scored kernels' 32 bits.
+bool scored_fits(int64_t N, int64_t vs2, int esz) {
+  return N <= (int64_t)1 << 22 && (N + 4096) * vs2 * esz < (int64_t)1 << 31;
 }
 
-// The launch shape of a launch over segments, or -1 where one workgroup
-// should walk every segment: a grid that leaves compute units idle, or whose
-// dim-split workgroups each stream every key (B = 1, N = 8192, D = 128: 31 us
-// by 64 workgroups of 8-way split dims, 16 us over 4 segments; B = 4: 55 and
-// 30 us; B = 16: 93 and 101 us). Short second segments are not worth the fold's
-// launch, about 2.5 us (N = 2100: 13 and 15 us; N = 3000: the same).
-int pick_split(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
-               int dtype, int mask_mode, int cus) {
-  if (dtype == BI_F32 || N <= kSegKeys + kSegKeys / 2) return -1;
+// The launch shape in which a problem takes the scores route, or -1 where one
+// workgroup per column (tile and slice of dims) does the whole: the route pays
+// where the walk along the keys is what takes the time and the grid leaves
+// compute units idle (one query row of one sequence, 32/8 heads, N = 8192,
+// keys and values in the last-level cache: D = 256 118 -> 28 us, D = 128
+// 26.0 -> 20.7, with an array mask 48 -> 28; in HBM 122 -> 41, 53 -> 31, 72 ->
+// 41), and not where a second launch and the scores' way through memory cost
+// more (8 sequences, D = 128: 41 and 50 us).
+// Both times, in microseconds, by least squares over a grid of H/Hkv = 32/8,
+// 8/8, 16/2, seven head-dim pairs, B = 1..16, 1..32 query rows, N = 512..16384
+// with and without an array mask (1470 problems, everything cached: from HBM
+// the route gains more); at 0.8 of the whole's estimate it was faster in every
+// one it took, and took nine tenths of those where it gains a tenth.
+int pick_scored(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
+                int dtype, int mask_mode, int cus) {
+  if (dtype == BI_F32 || N * D < 192 * 1024) return -1;
   const bool am = mask_mode == BI_MASK_ARRAY;
-  const int64_t streams = B * Hkv, ncol = (H / Hkv) * qL;
-  const int64_t tiles = streams * ((ncol + 15) / 16), ns = segments(N);
+  const int64_t streams = B * Hkv, ncol = H / Hkv * qL, tiles = streams * ((ncol + 15) / 16);
+  if (tiles > cus) return -1;
   const int walk = pick_shape(B, H, Hkv, qL, D, V, dtype, mask_mode, cus);
-  if (walk == SDPA_SHARED) return -1;
-  float best = estimate(D, V, tiles, streams, walk, am, 1, (float)N, (float)N, cus);
-  int shape = -1;
-  for (int s = SDPA_ROWS; s <= SDPA_SPLIT8; s++) {
-    if (s == SDPA_ROWS && (ncol <= 16 || sdpa_rows_tiles(D, V) != 2)) continue;
-    const float t = 1.05f * (2.5f + estimate(D, V, tiles, streams, s, am, ns, (float)N / (float)ns,
-                                             (float)kSegKeys, cus));
-    if (t < best) {
-      best = t;
-      shape = s;
-    }
-  }
-  return shape;
+  if (walk == SDPA_SHARED || (walk == SDPA_ROWS && sdpa_rows_tiles(D, V) == 2)) return -1;
+  if (scores_plan(B, H, Hkv, qL, N, D, cus).bytes > (int64_t)256 << 20) return -1;
+  // The most dim splits whose workgroups fit the compute units.
+  int shape = SDPA_TILE;
+  for (int s = SDPA_SPLIT2; s <= SDPA_SPLIT8; s++)
+    if (tiles * sdpa_shape_splits(V, s) <= cus) shape = s;
+  const float c = 1.f / (float)cus, d = (float)D, dw = (float)(V / sdpa_shape_splits(V, shape));
+  const float t = (float)tiles * c, wgs = t * (float)sdpa_shape_splits(V, shape);
+  const float hbm = (float)streams * c;  // streams per compute unit
+  const float scored = (am ? 6.68f + 0.0282f * dw : 2.18f + 0.0115f * dw) + 0.1245f * d * hbm +
+                       0.1227f * wgs * dw + 0.1555f * t * (float)(ncol < 16 ? ncol : 16) +
+                       (D > 256 ? 5.1f : 0.f);
+  const float vw = (float)V / (float)sdpa_shape_splits(V, walk);
+  const float whole = (am                                ? 2.48f + 0.1222f * d + 0.0112f * vw
+                       : sdpa_loaders(D, V, walk, false) ? 0.0441f * d + 0.0318f * t * (float)(D + V)
+                                                         : 0.1112f * d + 0.0044f * t * (float)(D + V)) +
+                      0.0337f * (float)(D + V) * hbm;
+  const float seg = (float)N / 2048.f;
+  return 8.1f + scored * seg < 0.8f * (3.73f + whole * seg) ? shape : -1;
 }
 
 // Validates, packs the arguments and launches shape `shape` (-1: the shape
-// bi_sdpa picks). `ws`, `ws_bytes`: memory for partial results, which lets a
-// launch take one segment of the keys per workgroup: with `split` it must
-// (shape says which), else it does where pick_split says so.
+// bi_sdpa picks). `ws`, `ws_bytes`: memory for raw scores; with `scored` the
+// launch takes them (shape says which it reads them in), else it does where
+// pick_scored says so.
 int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
              const int64_t* mask_strides, const void* sinks, void* out, int64_t B, int64_t H,
              int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
              const int64_t* qkv_strides, float scale, int mask_mode, int64_t causal_offset,
-             int dtype, int shape, bool split, void* ws, int64_t ws_bytes, void* hip_stream) {
+             int dtype, int shape, bool scored, void* ws, int64_t ws_bytes, void* hip_stream) {
   const int esz = bi::elem_size(dtype);
   if (!esz) return bi::fail(BI_EINVAL, "bi_sdpa: unknown dtype %d", dtype);
   if (B < 0 || H <= 0 || Hkv <= 0 || qL < 0 || N < 0 || D <= 0 || V <= 0)
@@ -636,21 +602,29 @@ int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
         ((H - 1) * p.ms[1] + (qL - 1) * p.ms[2] + N + kMaskSlack) * esz > INT32_MAX)
       return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: the mask of one batch entry is too large");
   }
-  p.part = nullptr;
-  p.nseg = 1;
-  if (split && (dtype == BI_F32 || shape == SDPA_SHARED))
-    return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: launch shape %d is not built over segments", shape);
-  const int64_t need = split_bytes(B, H, qL, N, V);
-  if (!split && shape < 0 && ws && ws_bytes >= need) {
-    shape = pick_split(B, H, Hkv, qL, N, D, V, dtype, mask_mode, device_cus());
-    split = shape >= 0;
+  p.sc = nullptr;
+  p.nsc = p.scw = p.bpw = 0;
+  if (scored && (dtype == BI_F32 || !scored_fits(N, p.vs[2], esz)))
+    return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: the scores route takes 16-bit types and streams "
+                    "below 2 GiB only");
+  if (!scored && shape < 0 && ws && dtype != BI_F32) {
+    shape = pick_scored(B, H, Hkv, qL, N, D, V, dtype, mask_mode, device_cus());
+    scored = shape >= 0 && scored_fits(N, p.vs[2], esz) &&
+             ws_bytes >= scores_plan(B, H, Hkv, qL, N, D, device_cus()).bytes;
+    if (!scored) shape = -1;
   }
-  if (split) {
-    if (!ws || (uintptr_t)ws % 16 || ws_bytes < need)
+  Scores sc = {};
+  if (scored && N > 0) {
+    sc = scores_plan(B, H, Hkv, qL, N, D, device_cus());
+    if (!ws || (uintptr_t)ws % 16 || ws_bytes < sc.bytes)
       return bi::fail(BI_EINVAL, "bi_sdpa: the workspace needs %lld bytes, 16-byte aligned",
-                      (long long)need);
-    p.part = static_cast<float*>(ws);
-    p.nseg = (int)segments(N);
+                      (long long)sc.bytes);
+    if (sc.blocks > INT32_MAX) return bi::fail(BI_EINVAL, "bi_sdpa: grid too large");
+    if (shape == SDPA_ROWS) shape = SDPA_TILE;  // built for one column tile
+    p.sc = static_cast<float*>(ws);
+    p.nsc = sc.nsc;
+    p.scw = sc.scw;
+    p.bpw = sc.bpw;
   }
   if (shape < 0) shape = pick_shape(B, H, Hkv, qL, D, V, dtype, mask_mode, device_cus());
   int columns = 0, splits = 0;
@@ -669,30 +643,29 @@ int sdpa_run(const void* q, const void* k, const void* v, const void* mask,
     blocks = rows / columns;
   } else {
     fn = mfma_kernel(D, V, dtype, mask_mode == BI_MASK_ARRAY, shape,
-                     split ? SEG_SPLIT : N > kSegKeys ? SEG_WALK : SEG_ONE);
+                     p.sc ? SDPA_SCORED : SDPA_WHOLE);
     const int64_t ncol = (H / Hkv) * qL;
-    blocks = B * Hkv * ((ncol + columns - 1) / columns) * splits * p.nseg;
+    blocks = B * Hkv * ((ncol + columns - 1) / columns) * splits;
   }
   if (blocks > INT32_MAX) return bi::fail(BI_EINVAL, "bi_sdpa: grid too large");
   if (!fn)
     return bi::fail(BI_EINVAL, "bi_sdpa: launch shape %d is not built for this mask", shape);
-  const int threads =
-      dtype == BI_F32 ? kThreads : sdpa_shape_threads(D, V, shape, mask_mode == BI_MASK_ARRAY);
+  const int threads = dtype == BI_F32 || p.sc
+                          ? kThreads
+                          : sdpa_shape_threads(D, V, shape, mask_mode == BI_MASK_ARRAY);
+  hipError_t e;
+  if (p.sc) {
+    const SdpaKernelFn sfn = mfma_kernel(D, V, dtype, false, sc.tiles, SDPA_SCORES);
+    if (!sfn) return bi::fail(BI_EUNSUPPORTED, "bi_sdpa: the scores route is not built here");
+    hipLaunchKernelGGL(sfn, dim3((unsigned)sc.blocks), dim3(kThreads), 0,
+                       static_cast<hipStream_t>(hip_stream), p);
+    e = hipGetLastError();
+    if (e != hipSuccess) return bi::launch_error(e, "bi_sdpa scores launch");
+  }
   hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3(threads), 0,
                      static_cast<hipStream_t>(hip_stream), p);
-  hipError_t e = hipGetLastError();
+  e = hipGetLastError();
   if (e != hipSuccess) return bi::launch_error(e, "bi_sdpa launch");
-  if (p.part) {
-    const int64_t fold_blocks = (rows * (V / 4) + 255) / 256;  // rows <= 2^31, V <= 512
-    if (dtype == BI_BF16)
-      hipLaunchKernelGGL(sdpa_fold_kernel<__bf16>, dim3((unsigned)fold_blocks), dim3(256), 0,
-                         static_cast<hipStream_t>(hip_stream), p, (int)V);
-    else
-      hipLaunchKernelGGL(sdpa_fold_kernel<_Float16>, dim3((unsigned)fold_blocks), dim3(256), 0,
-                         static_cast<hipStream_t>(hip_stream), p, (int)V);
-    e = hipGetLastError();
-    if (e != hipSuccess) return bi::launch_error(e, "bi_sdpa fold launch");
-  }
   return BI_OK;
 }
 
@@ -709,11 +682,11 @@ extern "C" int bi_sdpa(const void* q, const void* k, const void* v, const void* 
 
 extern "C" int64_t bi_sdpa_workspace(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N,
                                      int64_t D, int64_t V, int dtype, int mask_mode) {
-  if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || qL <= 0 || !dims_built(D, V)) return 0;
+  if (B <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || qL <= 0 || N <= 0 || !dims_built(D, V)) return 0;
   if (N > INT32_MAX - 1024 || B * H * qL > INT32_MAX) return 0;
-  return pick_split(B, H, Hkv, qL, N, D, V, dtype, mask_mode, device_cus()) < 0
-             ? 0
-             : split_bytes(B, H, qL, N, V);
+  const int cus = device_cus();
+  if (pick_scored(B, H, Hkv, qL, N, D, V, dtype, mask_mode, cus) < 0) return 0;
+  return scores_plan(B, H, Hkv, qL, N, D, cus).bytes;
 }
 
 extern "C" int bi_sdpa_ws(const void* q, const void* k, const void* v, const void* mask,

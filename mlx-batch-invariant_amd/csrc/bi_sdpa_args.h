@@ -24,20 +24,21 @@ struct SdpaArgs {
   uint32_t qsign;
   int mask_mode;
   int64_t causal_offset;
-  // SEG_SPLIT kernels: each workgroup takes one segment of kSegKeys keys (nseg
-  // of them) and leaves its columns' partial results here for
-  // sdpa_fold_kernel: O[column][segment][V], then (M, L)[column][segment],
-  // column = (b * H + head) * qL + row.
-  float* part;
-  int nseg;
+  // Raw scores in memory (SDPA_SCORES writes them, SDPA_SCORED reads them):
+  // per (stream, 16-column tile), nsc blocks of 32 keys, each the score
+  // MFMAs' results [kt][g][column < scw][e] of keys 16 kt + 4 g + e.
+  float* sc;
+  int nsc, scw;  // blocks per tile; columns kept per tile
+  int bpw;       // SDPA_SCORES: blocks per wave
 };
 
-// How a matrix-core kernel treats the segments of the keys: there is one
-// (N <= kSegKeys); its workgroups walk them all and fold them; or each
-// workgroup takes one and sdpa_fold_kernel folds them. The same arithmetic.
-enum SdpaSeg { SEG_ONE = 0, SEG_WALK = 1, SEG_SPLIT = 2 };
-// Keys per segment of the matrix-core kernels' fixed arithmetic.
-constexpr int kSegKeys = 2048;
+// What a matrix-core kernel does: the whole of a column; only its raw scores,
+// into SdpaArgs::sc (any number of workgroups along the keys); or the rest,
+// from those. A score depends on nothing but its query and key, so the two
+// together are the same arithmetic as the first.
+enum SdpaStage { SDPA_WHOLE = 0, SDPA_SCORES = 1, SDPA_SCORED = 2 };
+// Column tiles per workgroup of the scores kernel.
+constexpr int sdpa_score_tiles(int64_t D, int64_t ncol) { return ncol > 16 && D <= 256 ? 2 : 1; }
 
 typedef void (*SdpaKernelFn)(SdpaArgs);
 
@@ -105,8 +106,9 @@ constexpr int sdpa_shape_threads(int64_t D, int64_t V, int shape, bool array_mas
 }
 
 // The MFMA kernel of one head-dim pair for (dtype, array mask or not, shape,
-// SdpaSeg); nullptr where there is none (bi_sdpa_mfma_d*.hip).
+// SdpaStage; SDPA_SCORES: shape = column tiles per workgroup); nullptr where
+// there is none (bi_sdpa_mfma_d*.hip).
 #define BI_SDPA_MFMA_DECLARE(D, V) \
-  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int seg);
+  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int stage);
 BI_SDPA_DIM_PAIRS(BI_SDPA_MFMA_DECLARE)
 #undef BI_SDPA_MFMA_DECLARE

@@ -6,18 +6,17 @@
 // with matrix cores: one workgroup owns the whole key reduction for each of
 // its query columns -- a column is one (query head, query row) pair; the
 // columns of a workgroup share a batch index and a kv head, so they read the
-// same keys and values -- or, where the grid would leave the chip idle, one
-// segment of it, at fixed keys, its partial results folded by a second kernel
-// in the order the first would have. The workgroup's 4 waves walk the keys in a
+// same keys and values -- with no split-KV. (Raw scores, which depend on
+// nothing but their query and key, may come from a kernel that ran before:
+// SdpaStage, sdpa_scores_kernel and sdpa_scored_kernel.) The workgroup's 4 waves walk the keys in a
 // fixed stride order (the reference's fixed per-simdgroup strides, :89) and
 // their partial results are merged in a fixed order through LDS (:124-141).
 // D is the query/key head dim and V the value head dim (both multiples of 32,
 // reference :33-34, :224-227).
 //
 // Fixed per-column arithmetic (the invariance contract):
-//   * Keys are taken in segments of 2048 (fixed positions) and blocks of 32
-//     (block b = keys 32b .. 32b + 31). Block b belongs to chain b mod 4 of its
-//     segment; each chain walks its blocks in ascending order.
+//   * Keys are taken in blocks of 32 (block b = keys 32b .. 32b + 31). Block b
+//     belongs to chain b mod 4; each chain walks its blocks in ascending order.
 //   * Score: raw_i = q . k_i as a chain of v_mfma_f32_16x16x32_{bf16,f16}
 //     over the head dim in ascending 32-element chunks from +0.0 (exact
 //     products, fp32 sums). With a = |scale| * log2 e (a negative scale
@@ -25,7 +24,7 @@
 //     score is s_i = raw_i * a, plus mask_i * log2 e for an additive mask.
 //   * Key i is used iff i < N, i <= row + causal_offset (causal) and
 //     mask_i > -3e38 (array mask) (reference :92-96).
-//   * Each chain of a segment runs an online softmax in base 2 over its blocks: with M the
+//   * Each chain runs an online softmax in base 2 over its blocks: with M the
 //     largest used s_i of the block (without a mask taken as max_i(raw_i) * a,
 //     the same value since rounding is monotonic; none used: the block leaves
 //     the chain unchanged), m' = M > m + 8 ? M : m (a lazily moved base),
@@ -39,24 +38,15 @@
 //     keys 4g .. 4g + 3 and 16 + 4g .. 16 + 4g + 3. m starts at the lowest
 //     finite float and l at 0 (reference :76-79). A mask of zeros gives the
 //     bits of no mask.
-//   * A segment's chains merge in order: M = max of the chains' m; L = 0,
-//     O = +0.0; then for c = 0, 1, 2, 3, e_c = exp2(m_c - M),
-//     L = fma(l_c, e_c, L) and O = fma(o_c, e_c, O). A sink (reference :80-86,
-//     an extra denominator term exp(sink)) enters the first segment's merge as
-//     one more partial with m = sink * log2 e, l = 1, o = 0, ahead of the
-//     chains: M is the max with it too, and L starts at exp2(sink2 - M).
+//   * Merge: a sink (reference :80-86, an extra denominator term exp(sink))
+//     enters here as one more partial with m = sink * log2 e, l = 1, o = 0,
+//     ahead of the chains: M = max of the sink's and the chains' m;
+//     L = exp2(sink2 - M) (0 without a sink), O = +0.0; then for
+//     c = 0, 1, 2, 3 in order, e_c = exp2(m_c - M), L = fma(l_c, e_c, L) and
+//     O = fma(o_c, e_c, O); O = O + 0.0 (a product that underflows from below
+//     leaves -0.0); out = L == 0 ? O : O / L, one rounding to T.
 //     (Seeding a chain's base with the sink, as the reference seeds its
 //     simdgroup 0, would put a large sink's p below f16's range.)
-//   * The segments fold in ascending order: the first segment's (M, L, O) is
-//     the running (R, S, Q); then R' = max(R, M), e = exp2(R - R'),
-//     f = exp2(M - R'), S = fma(L, f, S * e), Q = fma(O, f, Q * e) + 0.0.
-//     out = S == 0 ? Q : Q / S, one rounding to T, of Q + 0.0 where there is
-//     one segment: a product that underflows from below leaves -0.0, which
-//     the addition turns into +0.0, so Q is never -0.0, a segment without a
-//     usable key (f == 0 or O == 0) changes no bit of it, and neither does
-//     the number of such segments or which of them a launch skips.
-//     Segments lie at fixed keys, so whether one workgroup walks them all or
-//     each has its own workgroup changes nothing a column computes.
 // Every column, whatever workgroup or lane it lands in, however many rows or
 // heads share its keys and whatever the launch shape (columns per workgroup,
 // prefetch depths), runs exactly this sequence: an output row has the same
@@ -72,7 +62,6 @@
 
 #include "bi_internal.h"
 #include "bi_sdpa_args.h"
-#include "bi_sdpa_fold.h"
 
 namespace {
 
@@ -80,6 +69,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 f16x4_t __attribute__((ext_vector_type(4)));
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(3))) i16x4_t lds_i16x4_t;
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -97,8 +87,7 @@ __device__ __forceinline__ void st16(uint4* p, uint4 v) {
 constexpr int kWaves = 4;  // = chains
 constexpr int kThreads = 64 * kWaves;
 constexpr int kBlk = 32;   // keys per block
-constexpr int kSegBlk = kSegKeys / kBlk;      // blocks per segment
-constexpr int kSegIt = kSegBlk / kWaves;      // of them in one chain
+constexpr float kLog2e = 1.4426950408889634f;
 
 // s_waitcnt immediates (gfx9 encoding: vmcnt [3:0] + [15:14], expcnt [6:4],
 // lgkmcnt [11:8]).
@@ -158,13 +147,6 @@ __device__ __forceinline__ u32x4_t ds_read_b128_at(uint32_t lds_addr, int off) {
   u32x4_t v;
   asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(lds_addr), "i"(off) : "memory");
   return v;
-}
-
-// A 16-byte LDS write of matrix-product results as an asm statement. The
-// compiler does not count the wait states between an MFMA and an asm
-// statement that reads its result; 24 cover every MFMA used here.
-__device__ __forceinline__ void ds_write_acc(uint32_t lds_addr, f32x4_t v) {
-  asm volatile("s_nop 15\n\ts_nop 7\n\tds_write_b128 %0, %1" ::"v"(lds_addr), "v"(v) : "memory");
 }
 
 template <typename T> __device__ inline unsigned short tbits(T x) {
@@ -315,7 +297,7 @@ struct Chain {
   const T* mb;
   int64_t ks2, vs2, N, mext;
   int nit;
-  int wave;  // the chain's first block (block i of the chain: wave + 4i)
+  int wave;
   // Lane byte offsets: key row 16kt + r16 at dims 8g ..; value chunk j;
   // mask keys 4g .. of the lane's row in each column tile. The other key and
   // mask loads add constants (immediate offsets, which the range check
@@ -427,8 +409,8 @@ struct Chain {
 // LW: 0, or kWaves loader waves (keys in LDS only). A loader wave issues the
 // loads of one chain's blocks, so the chain wave's instruction stream holds
 // no load issue (which stalls while the memory pipeline is busy).
-template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
-__device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
+template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW>
+__global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs p) {
   static_assert(LW == 0 || (LW == kWaves && KL && PK == 0 && SV >= 3), "loader waves: one per chain");
   using C = Chain<T, D, V, CT, PK, SV, WS, MK, KL>;
   constexpr int NQ = C::NQ, NB = C::NB, VCH = C::VCH;
@@ -454,15 +436,9 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
   const int64_t G = p.H / p.Hkv;
   const int64_t ncol = G * p.qL;
   const int64_t ncb = (ncol + COLS - 1) / COLS;
-  const int nsplit = SEG == SEG_SPLIT ? p.nseg : 1;
-  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * ncb * WS * nsplit));
+  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * ncb * WS));
   const int ws = (int)(t % WS);
   t /= WS;
-  int seg = 0;  // SEG_SPLIT: this workgroup's
-  if constexpr (SEG == SEG_SPLIT) {
-    seg = (int)(t % nsplit);
-    t /= nsplit;
-  }
   // Causal: the last column blocks see the most keys; they start first.
   const int64_t cb = p.mask_mode == BI_MASK_CAUSAL ? ncb - 1 - t % ncb : t % ncb;
   t /= ncb;
@@ -481,12 +457,7 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
   const int64_t kmax = kend_of(last_cc / G);  // keys some column of the workgroup sees
   // Block counts and indices fit in 32 bits (the host bounds N below
   // 2^31 - 1024), which keeps the loop's compares on the scalar unit.
-  // This workgroup's blocks: blk0 .. blk0 + nblk - 1, in nsg segments.
-  const int blk0 = seg * kSegBlk;
-  int nblk = (int)((kmax + kBlk - 1) / kBlk);
-  if constexpr (SEG == SEG_SPLIT)
-    nblk = nblk <= blk0 ? 0 : nblk - blk0 < kSegBlk ? nblk - blk0 : kSegBlk;
-  const int nsg = SEG == SEG_WALK ? (nblk + kSegBlk - 1) / kSegBlk : 1;
+  const int nblk = (int)((kmax + kBlk - 1) / kBlk);
   const int nfull = (int)(kend_of(c0 / G) / kBlk);  // blocks every column of the workgroup sees
 
   // This lane's column in each tile; its query as the B operand of the score
@@ -519,11 +490,11 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
   // Key and value rows of the stream; per-block buffer resources start at the
   // block's first row, so the lane offsets below are the same for every block
   // (and below 2^31: the host bounds 32 * stride).
-  // This chain's blocks are blk0 + wave + 4i, i < nit.
+  // This chain's blocks are wave + 4i, i < nit.
   const int nit = nblk > wave ? (nblk - wave + kWaves - 1) / kWaves : 0;
   const int wslot = wave * C::VSLOT;  // this wave's slot within each array
   C ld;
-  ld.init(p, b, kvh, ws, blk0 + wave, nit, lane, mrow, kmax);
+  ld.init(p, b, kvh, ws, wave, nit, lane, mrow, kmax);
   // With loader waves every wave runs the same number of steps (chain 0 has
   // the most blocks), one barrier each. PIPE (four slots or more): at step j
   // a chain wave reads and scores the keys of block j while it finishes block
@@ -534,11 +505,6 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
   constexpr bool PIPE = LW != 0 && SV >= 4;
   constexpr int AHEAD = PIPE ? SV - 2 : SV - 1;
   const int steps = PIPE ? nit0 + 1 : nit0;
-  // Whether each chain's first n blocks end a segment that another follows:
-  // the chains then merge before the next (one more barrier with loader waves).
-  auto ends_segment = [&](int n) __attribute__((always_inline)) -> bool {
-    return SEG == SEG_WALK && n % kSegIt == 0 && n > 0 && n < nsg * kSegIt;
-  };
   if constexpr (LW != 0) {
     if (loader) {
       // Block j lands in slot j % SV. Before barrier j this wave waits for
@@ -556,7 +522,6 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
           __builtin_amdgcn_s_waitcnt(wait_vm((AHEAD - 1) * (C::DK + C::DV)));
           asm volatile("s_barrier" ::: "memory");
           ld.vload(j0 + u + AHEAD, arr((u + AHEAD) % SV) + wslot);
-          if (ends_segment(PIPE ? j0 + u : j0 + u + 1)) asm volatile("s_barrier" ::: "memory");
         }
       }
       // The merge below reuses the slots: no load may still be landing
@@ -799,148 +764,6 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
     update(std::false_type{}, sc, mk, slot, blk, va);
   };
 
-  // The running state over the segments so far: (R, S) of each column, and Q
-  // of the dim blocks wave, wave + 4, ... this wave writes out. With two
-  // column tiles, Q lives in LDS between its uses, once in 2048 keys, where
-  // two workgroups' LDS allows, and else all of it in scratch memory
-  // (volatile): two such workgroups share a CU, and their chains' state fills
-  // the 256 registers that leaves a wave.
-  constexpr int KB = (NB + kWaves - 1) / kWaves;
-  constexpr bool QLDS = CT == 2 && SEG == SEG_WALK &&
-                        SV * C::ARR_U4 * 16 + CT * kWaves * KB * 1024 + 1024 <= 80 * 1024;
-  constexpr bool RMEM = CT == 2 && SEG == SEG_WALK && !QLDS;
-  struct Run {
-    float R, S;
-    f32x4_t Q[KB];
-  };
-  volatile float rmem[RMEM ? CT * (2 + 4 * KB) : 1];
-  auto qmem = []() __attribute__((always_inline)) -> uint4* {
-    if constexpr (QLDS) {
-      __shared__ uint4 q[CT * kWaves * KB * 64];
-      return q;
-    }
-    return nullptr;
-  };
-  Run rreg[CT];
-  auto run_get = [&](int ct, bool first, Run& r) __attribute__((always_inline)) {
-    if (SEG != SEG_WALK || first) {  // the fold of the first segment leaves it as it is
-      r.R = -FLT_MAX;
-      r.S = 0.f;
-#pragma unroll
-      for (int k = 0; k < KB; k++) r.Q[k] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    } else if constexpr (RMEM) {
-      r.R = rmem[ct * (2 + 4 * KB)];
-      r.S = rmem[ct * (2 + 4 * KB) + 1];
-#pragma unroll
-      for (int k = 0; k < KB; k++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) r.Q[k][e] = rmem[ct * (2 + 4 * KB) + 2 + 4 * k + e];
-    } else if constexpr (QLDS) {
-      r.R = rreg[ct].R;
-      r.S = rreg[ct].S;
-#pragma unroll
-      for (int k = 0; k < KB; k++)
-        r.Q[k] = __builtin_bit_cast(f32x4_t, ld16(qmem() + ((ct * kWaves + wave) * KB + k) * 64 + lane));
-    } else {
-      r = rreg[ct];
-    }
-  };
-  auto run_put = [&](int ct, const Run& r) __attribute__((always_inline)) {
-    if constexpr (RMEM) {
-      rmem[ct * (2 + 4 * KB)] = r.R;
-      rmem[ct * (2 + 4 * KB) + 1] = r.S;
-#pragma unroll
-      for (int k = 0; k < KB; k++)
-#pragma unroll
-        for (int e = 0; e < 4; e++) rmem[ct * (2 + 4 * KB) + 2 + 4 * k + e] = r.Q[k][e];
-    } else if constexpr (QLDS) {
-      rreg[ct].R = r.R;
-      rreg[ct].S = r.S;
-#pragma unroll
-      for (int k = 0; k < KB; k++)
-        st16(qmem() + ((ct * kWaves + wave) * KB + k) * 64 + lane, __builtin_bit_cast(uint4, r.Q[k]));
-    } else {
-      rreg[ct] = r;
-    }
-  };
-  static_assert(CT <= 2, "running state of one or two column tiles");
-  // A segment's end inside the walk: the chains exchange (m, l, o) through
-  // this wave's part of value slot `slot`, whose block has been used and
-  // whose refill the caller orders behind the readers; the loads of the next
-  // blocks stay in flight (asm LDS accesses, see ds_read_tr).
-  auto mls = []() __attribute__((always_inline)) -> float2* {
-    if constexpr (!KL && SEG == SEG_WALK) {
-      __shared__ float2 ml[kWaves * 16];
-      return ml;
-    }
-    return nullptr;
-  };
-  auto mid_merge = [&](int slot, bool first) __attribute__((always_inline)) {
-    const uint32_t ob = (uint32_t)(uintptr_t)(lds_void_t*)(arr(slot) + C::KSLOT) + lane * 16;
-    // (m, l) of a column, which its four lanes all hold.
-    const uint32_t mb = KL ? (uint32_t)(uintptr_t)(lds_void_t*)arr(slot) + r16 * 8
-                           : (uint32_t)(uintptr_t)(lds_void_t*)mls() + r16 * 8;
-    constexpr uint32_t MS = KL ? C::VSLOT * 16 : 16 * 8;  // bytes between the chains' (m, l)
-#pragma unroll
-    for (int ct = 0; ct < CT; ct++) {
-      if (ct > 0) asm volatile("s_barrier" ::: "memory");  // the last tile's readers
-#pragma unroll
-      for (int db = 0; db < NB; db++) ds_write_acc(ob + (wslot + db * 64) * 16, o[ct][db]);
-      const f32x2_t mv = {m[ct], l[ct]};
-      asm volatile("ds_write_b64 %0, %1" ::"v"(mb + wave * MS), "v"(mv) : "memory");
-      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-      u32x2_t sv[kWaves];
-      u32x4_t ov[KB][kWaves];
-#pragma unroll
-      for (int c = 0; c < kWaves; c++)
-        asm volatile("ds_read_b64 %0, %1" : "=v"(sv[c]) : "v"(mb + c * MS) : "memory");
-#pragma unroll
-      for (int k = 0; k < KB; k++) {
-        const int db = wave + kWaves * k < NB ? wave + kWaves * k : 0;
-#pragma unroll
-        for (int c = 0; c < kWaves; c++) ov[k][c] = ds_read_b128(ob + (c * C::VSLOT + db * 64) * 16);
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-      for (int c = 0; c < kWaves; c++) {
-        asm volatile("" : "+v"(sv[c]));
-#pragma unroll
-        for (int k = 0; k < KB; k++) asm volatile("" : "+v"(ov[k][c]));
-      }
-      float ec[kWaves];
-      const float sk = first && p.sinks ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e
-                                        : -FLT_MAX;
-      float M = sk;
-#pragma unroll
-      for (int c = 0; c < kWaves; c++) M = fmaxf(M, __uint_as_float(sv[c][0]));
-      float L = first && p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
-#pragma unroll
-      for (int c = 0; c < kWaves; c++) {
-        ec[c] = __builtin_amdgcn_exp2f(__uint_as_float(sv[c][0]) - M);
-        L = __builtin_fmaf(__uint_as_float(sv[c][1]), ec[c], L);
-      }
-      Run r;
-      run_get(ct, first, r);
-      const FoldW w = fold_stats(r.R, r.S, M, L);
-#pragma unroll
-      for (int k = 0; k < KB; k++) {
-        f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int c = 0; c < kWaves; c++) {
-          const f32x4_t oc = __builtin_bit_cast(f32x4_t, ov[k][c]);
-#pragma unroll
-          for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
-        }
-        fold_out(r.Q[k], O, w);
-      }
-      run_put(ct, r);
-      m[ct] = -FLT_MAX;
-      l[ct] = 0.f;
-#pragma unroll
-      for (int i = 0; i < NB; i++) o[ct][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-
   // Block i of the chain: keys loaded at step i - PK, values at step
   // i - SV + 1 into slot i % SV. The loop is unrolled over U steps (the
   // least common multiple of the two rotations) so that register and slot
@@ -970,11 +793,7 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
           // their latency.
           VA_t va;
           vread((u + SV - 1) % SV, va);
-          update(std::true_type{}, sp, kr[0].m, (u + SV - 1) % SV, blk0 + wave + kWaves * (j - 1), va);
-        }
-        // (Barrier j + 1 precedes the slot's refill.)
-        if constexpr (SEG == SEG_WALK) {
-          if (ends_segment(j)) mid_merge((u + SV - 1) % SV, j == kSegIt);
+          update(std::true_type{}, sp, kr[0].m, (u + SV - 1) % SV, wave + kWaves * (j - 1), va);
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         scores(kr[0], kl, sp);
@@ -988,10 +807,7 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
         const int j = j0 + u;
         if (j >= steps) break;
         asm volatile("s_barrier" ::: "memory");
-        if (j < nit) compute(kr[0], kr[0].m, u, blk0 + wave + kWaves * j);
-        if constexpr (SEG == SEG_WALK) {  // (barrier j + 1 precedes the slot's refill)
-          if (ends_segment(j + 1)) mid_merge(u, j + 1 == kSegIt);
-        }
+        if (j < nit) compute(kr[0], kr[0].m, u, wave + kWaves * j);
       }
     }
   } else {
@@ -999,8 +815,7 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
     for (int u = 0; u < SV - 1; u++) ld.vload(u, arr(u) + wslot);
 #pragma unroll
     for (int u = 0; u < PK; u++) ld.kload(u, kr[u]);
-    static_assert(kSegIt % U == 0, "segments end on a round of the loop");
-    for (int i0 = 0; i0 < (SEG == SEG_WALK ? nit0 : nit); i0 += U) {
+    for (int i0 = 0; i0 < nit; i0 += U) {
 #pragma unroll
       for (int u = 0; u < U; u++) {
         const int i = i0 + u;
@@ -1009,21 +824,17 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
         ld.vload(i + SV - 1, arr((u + SV - 1) % SV) + wslot);
         if (i < nit) {
           if constexpr (MK == 2)
-            compute(kr[u % (PK + 1)], mcur.m, u % SV, blk0 + wave + kWaves * i);
+            compute(kr[u % (PK + 1)], mcur.m, u % SV, wave + kWaves * i);
           else
-            compute(kr[u % (PK + 1)], kr[u % (PK + 1)].m, u % SV, blk0 + wave + kWaves * i);
-        }
-        if (SEG == SEG_WALK && u == U - 1 && ends_segment(i + 1)) {
-          mid_merge(u % SV, i + 1 == kSegIt);
-          asm volatile("s_barrier" ::: "memory");  // the slot's readers, before its refill
+            compute(kr[u % (PK + 1)], kr[u % (PK + 1)].m, u % SV, wave + kWaves * i);
         }
       }
     }
   }
 
-  // The last segment's merge, one column tile at a time: o of chain c in va0,
-  // (m, l) in va1 (the value slots are free once every wave's loads and reads
-  // have completed); then its fold and the output, or the partial result.
+  // Merge the 4 chains in order through LDS, one column tile at a time: o of
+  // chain c in va0, (m, l) in va1 (the value slots are free once every
+  // wave's loads and reads have completed).
   uint4* const mo = va0;
   float2* const ml = reinterpret_cast<float2*>(va1);
 #pragma unroll
@@ -1038,8 +849,7 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
     asm volatile("s_barrier" ::: "memory");
     float mc[kWaves], lc[kWaves], ec[kWaves];
     // The sink (base 2) first: -FLT_MAX without one.
-    const bool sink = p.sinks && (SEG == SEG_ONE || (SEG == SEG_WALK ? nsg <= 1 : seg == 0));
-    const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e : -FLT_MAX;
+    const float sk = p.sinks ? (float)static_cast<const T*>(p.sinks)[head[ct]] * kLog2e : -FLT_MAX;
     float M = sk;
 #pragma unroll
     for (int c = 0; c < kWaves; c++) {
@@ -1048,29 +858,17 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
       lc[c] = v.y;
       M = fmaxf(M, mc[c]);
     }
-    float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
+    float L = p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
 #pragma unroll
     for (int c = 0; c < kWaves; c++) {
       ec[c] = __builtin_amdgcn_exp2f(mc[c] - M);
       L = __builtin_fmaf(lc[c], ec[c], L);
     }
-    const int64_t col = (b * p.H + head[ct]) * p.qL + srow[ct];
-    Run r;
-    FoldW w = {0.f, 0.f};
-    if constexpr (SEG == SEG_WALK) {
-      run_get(ct, nsg <= 1, r);
-      w = fold_stats(r.R, r.S, M, L);
-      L = r.S;
-    }
-    if constexpr (SEG == SEG_SPLIT) {
-      if (colv[ct] && ws == 0 && wave == 0 && g == 0)
-        *reinterpret_cast<float2*>(p.part + p.B * p.H * p.qL * p.nseg * V + (col * p.nseg + seg) * 2) =
-            make_float2(M, L);
-    }
-    T* __restrict__ out = static_cast<T*>(p.out) + col * V + ws * C::DW;
+    T* __restrict__ out =
+        static_cast<T*>(p.out) + ((b * p.H + head[ct]) * p.qL + srow[ct]) * V + ws * C::DW;
     // Wave w writes out the dim blocks w, w + 4, ... of this workgroup.
 #pragma unroll
-    for (int k = 0; k < KB; k++) {
+    for (int k = 0; k < (NB + kWaves - 1) / kWaves; k++) {
       const int db = wave + kWaves * k;
       if (db >= NB) break;
       f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -1080,36 +878,483 @@ __device__ __forceinline__ void sdpa_mfma_body(SdpaArgs p) {
 #pragma unroll
         for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
       }
-      if constexpr (SEG == SEG_SPLIT) {
-        float* __restrict__ part = p.part + (col * p.nseg + seg) * V + ws * C::DW;
-        if (colv[ct]) *reinterpret_cast<f32x4_t*>(part + 16 * db + 4 * g) = O;
-      } else {
-        if constexpr (SEG == SEG_WALK) {
-          fold_out(r.Q[k], O, w);
-          O = r.Q[k];
-        } else {
-          O += 0.f;
-        }
-        unsigned short ob[4];
+      O += 0.f;
+      unsigned short ob[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
-        if (colv[ct])
-          *reinterpret_cast<uint2*>(out + 16 * db + 4 * g) =
-              make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
-      }
+      for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
+      if (colv[ct])
+        *reinterpret_cast<uint2*>(out + 16 * db + 4 * g) =
+            make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
     }
   }
 }
 
-template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
-__global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs p) {
-  sdpa_mfma_body<T, D, V, CT, PK, SV, WS, MK, KL, LW, SEG>(p);
+// SDPA_SCORES: the raw scores of CTS column tiles against blocks of 32 keys,
+// into SdpaArgs::sc. A wave takes every fourth of its workgroup's 4 * bpw
+// consecutive blocks, the next one's keys in flight; no block depends on
+// another, so the grid can fill the chip whatever the number of streams.
+// Keys no column of the stream can see read as zeros. Bound by the latency of
+// one or two rounds of loads per wave: 16.8 MB of keys (one sequence, 8 kv
+// heads, D = 128, N = 8192) from HBM 7.1 us, 4.2 MB 3.9 us.
+template <typename T, int D, int CTS>
+__global__ void __launch_bounds__(kThreads) sdpa_scores_kernel(SdpaArgs p) {
+  constexpr int NQ = D / 32;
+  constexpr uint32_t E = sizeof(T);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, r16 = lane & 15;
+  // Workgroup -> (batch, kv head, run of blocks, group of column tiles): the
+  // groups that read the same keys are neighbours.
+  const int64_t G = p.H / p.Hkv;
+  const int64_t ncol = G * p.qL;
+  const int64_t ncb = (ncol + 15) / 16, ntg = (ncb + CTS - 1) / CTS;
+  const int64_t nch = (p.nsc + kWaves * p.bpw - 1) / (kWaves * p.bpw);
+  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * nch * ntg));
+  const int64_t tg = t % ntg;
+  t /= ntg;
+  const int64_t ch = t % nch;
+  t /= nch;
+  const int64_t kvh = t % p.Hkv;
+  const int64_t b = t / p.Hkv;
+
+  int64_t nk = p.N;  // keys that the last row sees
+  if (p.mask_mode == BI_MASK_CAUSAL) {
+    const int64_t last = p.qL - 1 + p.causal_offset;
+    nk = last < 0 ? 0 : (last + 1 < p.N ? last + 1 : p.N);
+  }
+  uint4 qt[CTS][NQ];
+  float* dst[CTS];
+#pragma unroll
+  for (int ct = 0; ct < CTS; ct++) {
+    const int64_t cb = tg * CTS + ct, cc = cb * 16 + r16;
+    const bool colv = cc < ncol;
+    const int64_t row = colv ? cc / G : 0, head = kvh * G + (colv ? cc % G : 0);
+    const T* qrow = static_cast<const T*>(p.q) + b * p.qs[0] + head * p.qs[1] + row * p.qs[2];
+#pragma unroll
+    for (int i = 0; i < NQ; i++)
+      qt[ct][i] = colv ? qneg(ld16(qrow + 32 * i + 8 * g), p.qsign) : make_uint4(0, 0, 0, 0);
+    dst[ct] = cb < ncb && r16 < p.scw
+                  ? p.sc + ((b * p.Hkv + kvh) * ncb + cb) * p.nsc * (int64_t)(kBlk * p.scw) +
+                        (g * p.scw + r16) * 4
+                  : nullptr;
+  }
+  const T* kb = static_cast<const T*>(p.k) + b * p.ks[0] + kvh * p.ks[1];
+  const int64_t ks2 = p.ks[2];
+  uint32_t koff[2];
+#pragma unroll
+  for (int kt = 0; kt < 2; kt++) koff[kt] = (uint32_t)(((16 * kt + r16) * ks2 + 8 * g) * E);
+  const int64_t blk0 = ch * kWaves * p.bpw + wave;
+  auto load = [&](int j, uint4 (&kr)[2][NQ]) __attribute__((always_inline)) {
+    const int64_t key0 = (blk0 + kWaves * j) * kBlk;
+    const bool in = j < p.bpw && key0 < nk;
+    const auto rs = make_rsrc_n(kb + (in ? key0 * ks2 : 0),
+                                in ? clamp31(((nk - key0 - 1) * ks2 + D) * (int64_t)E) : 0u);
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int q = 0; q < NQ; q++)
+        kr[kt][q] = __builtin_bit_cast(
+            uint4, __builtin_amdgcn_raw_buffer_load_b128(rs, (int)(koff[kt] + 32 * q * E), 0, 0));
+  };
+  auto block = [&](int j, const uint4 (&kr)[2][NQ]) __attribute__((always_inline)) {
+    const int64_t blk = blk0 + kWaves * j;
+    if (j >= p.bpw || blk >= p.nsc) return;
+#pragma unroll
+    for (int ct = 0; ct < CTS; ct++)
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++) {
+        f32x4_t s = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NQ; i++) s = mma32(T(0), kr[kt][i], qt[ct][i], s);
+        if (dst[ct])
+          *reinterpret_cast<f32x4_t*>(dst[ct] + blk * (kBlk * p.scw) + 16 * kt * p.scw) = s;
+      }
+  };
+  uint4 kr[2][2][NQ];
+  load(0, kr[0]);
+  for (int j = 0; j < p.bpw; j += 2) {
+    load(j + 1, kr[1]);
+    block(j, kr[0]);
+    load(j + 2, kr[0]);
+    block(j + 1, kr[1]);
+  }
 }
-// The same with the registers of as many waves per SIMD (two, or three for
-// heads up to 64) as the two-tile kernels of one segment leave room for.
-template <typename T, int D, int V, int CT, int PK, int SV, int WS, int MK, bool KL, int LW, int SEG>
-__global__ void __launch_bounds__(kThreads + 64 * LW, D + V <= 128 ? 3 : 2) sdpa_mfma_kernel2(SdpaArgs p) {
-  sdpa_mfma_body<T, D, V, CT, PK, SV, WS, MK, KL, LW, SEG>(p);
+
+// SDPA_SCORED: sdpa_mfma_kernel's one-tile shapes with the scores already in
+// memory: the same operations on the same values in the same order from there
+// on. A chain's step is then its softmax and the P.V products alone, short
+// beside the latency of memory: scores (and mask values) are loaded SV - PB
+// blocks ahead into registers and values into slots, by offsets that only grow
+// (one addition each; past the end they read zeros), and the softmaxes of PB
+// blocks run side by side where no base moves in them. Bound by the softmax's
+// issue (0.2 us a block with everything cached) and, from HBM, by the loads in
+// flight (0.3 us): one sequence, 32/8 heads, N = 8192, D = 128, 8-way split
+// dims 21.8 us from HBM (23.6 one block at a time), where the whole takes 52.
+template <typename T, int V, int WS, bool MASK>
+struct ScoredLoads {
+  using C = Chain<T, 32, V, 1, 1, 2, WS, 0, false>;  // the value slots' layout
+  static constexpr int DV = C::DV;
+  static constexpr uint32_t E = sizeof(T);
+  // The tile's scores, the stream's values (up to the last key that some
+  // column sees) and the batch's mask, and their bytes (the host bounds the
+  // lane offsets, and some blocks more, below 2^32).
+  const float* sc;
+  const T* v;
+  const T* mask;
+  uint32_t sn, vn, mn;
+  uint32_t sstep, vstep;  // bytes from a block of the chain to its next
+  uint32_t so[2], vo[DV], mo;
+  __device__ __forceinline__ void init(const SdpaArgs& p, int64_t b, int64_t kvh, int ws,
+                                       int64_t tile, int64_t kmax, int64_t head, int64_t srow,
+                                       int wave, int lane) {
+    const int g = lane >> 4, r16 = lane & 15;
+    const uint32_t scs = (uint32_t)(kBlk * p.scw * 4), vs = (uint32_t)(p.vs[2] * kBlk * E);
+    sc = p.sc + tile * p.nsc * (int64_t)(kBlk * p.scw);
+    sn = (uint32_t)p.nsc * scs;
+    v = static_cast<const T*>(p.v) + b * p.vs[0] + kvh * p.vs[1];
+    vn = kmax > 0 ? (uint32_t)(((kmax - 1) * p.vs[2] + V) * E) : 0u;
+    sstep = kWaves * scs;
+    vstep = kWaves * vs;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)  // (a column that is not kept: past the end)
+      so[kt] = r16 < p.scw ? (uint32_t)(((4 * kt + g) * p.scw + r16) * 16) + wave * scs : 0x80000000u;
+#pragma unroll
+    for (int j = 0; j < DV; j++) {
+      const int pos = j * 64 + lane, r = pos / C::VCH, c = C::vchunk_src(r, pos % C::VCH);
+      vo[j] = (uint32_t)((r * p.vs[2] + ws * C::DW + c * 8) * E) + wave * vs;
+    }
+    if constexpr (MASK) {
+      mask = static_cast<const T*>(p.mask) + b * p.ms[0];
+      mn = (uint32_t)(((p.H - 1) * p.ms[1] + (p.qL - 1) * p.ms[2] + p.N) * E);
+      mo = (uint32_t)((head * p.ms[1] + srow * p.ms[2] + 4 * g + wave * kBlk) * E);
+    }
+  }
+  // The chain's next block (in order): scores and mask values; values.
+  __device__ __forceinline__ void sload(f32x4_t (&s)[2], unsigned short (&mk)[8]) {
+    const auto rs = make_rsrc_n(sc, sn);
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      s[kt] = __builtin_bit_cast(f32x4_t,
+                                 __builtin_amdgcn_raw_buffer_load_b128(rs, (int)so[kt], 0, 0));
+      so[kt] += sstep;
+    }
+    if constexpr (MASK) {
+      const auto rm = make_rsrc_n(mask, mn);
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+        mk[j] = __builtin_amdgcn_raw_buffer_load_b16(
+            rm, (int)(mo + (16 * (j >> 2) + (j & 3)) * E), 0, 0);
+      mo += kWaves * kBlk * E;
+    }
+  }
+  __device__ __forceinline__ void vload(uint4* dst) {
+    const auto rv = make_rsrc_n(v, vn);
+#pragma unroll
+    for (int j = 0; j < DV; j++) {
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_void_t*)(dst + j * 64), 16, (int)vo[j], 0, 0,
+                                               0);
+      vo[j] += vstep;
+    }
+  }
+};
+
+template <typename T, int V, int SV, int PB, int WS, bool MASK>
+__global__ void __launch_bounds__(kThreads) sdpa_scored_kernel(SdpaArgs p) {
+  using Loads = ScoredLoads<T, V, WS, MASK>;
+  using C = typename Loads::C;
+  constexpr int NB = C::NB, VCH = C::VCH, DV = C::DV;
+  constexpr int VWAIT = (SV - PB) * (2 + (MASK ? 8 : 0) + DV);
+  static_assert(SV > PB && SV % PB == 0 && VWAIT <= 63, "loads in flight exceed the vmcnt range");
+  static_assert(SV * C::ARR_U4 * 16 <= 160 * 1024, "LDS per workgroup");
+  __shared__ uint4 va[SV * C::ARR_U4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the chain
+  const int g = lane >> 4, r16 = lane & 15;
+
+  const int64_t G = p.H / p.Hkv;
+  const int64_t ncol = G * p.qL;
+  const int64_t ncb = (ncol + 15) / 16;
+  int64_t t = xcd_remap(blockIdx.x, (int)(p.B * p.Hkv * ncb * WS));
+  const int ws = (int)(t % WS);
+  t /= WS;
+  const int64_t cb = p.mask_mode == BI_MASK_CAUSAL ? ncb - 1 - t % ncb : t % ncb;
+  t /= ncb;
+  const int64_t kvh = t % p.Hkv;
+  const int64_t b = t / p.Hkv;
+  const int64_t c0 = cb * 16;
+  auto kend_of = [&](int64_t s) __attribute__((always_inline)) -> int64_t {
+    if (p.mask_mode != BI_MASK_CAUSAL) return p.N;
+    const int64_t last = s + p.causal_offset;
+    return last < 0 ? 0 : (last + 1 < p.N ? last + 1 : p.N);
+  };
+  const int64_t last_cc = (c0 + 16 < ncol ? c0 + 16 : ncol) - 1;
+  const int64_t kmax = kend_of(last_cc / G);
+  const int nblk = (int)((kmax + kBlk - 1) / kBlk);
+  const int nfull = MASK ? 0 : (int)(kend_of(c0 / G) / kBlk);
+  const int nit = nblk > wave ? (nblk - wave + kWaves - 1) / kWaves : 0;
+  const int nfit = nfull > wave ? (nfull - wave + kWaves - 1) / kWaves : 0;  // full ones
+
+  const int64_t cc = c0 + r16;
+  const bool colv = cc < ncol;
+  const int64_t srow = colv ? cc / G : 0, head = kvh * G + (colv ? cc % G : 0);
+  const int kend = colv ? (int)kend_of(srow) : 0;
+  float m = -FLT_MAX, l = 0.f;
+  f32x4_t o[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  Loads ld;
+  ld.init(p, b, kvh, ws, (b * p.Hkv + kvh) * ncb + cb, kmax, head, srow, wave, lane);
+  // Values of a block transposed for the P.V products: the lane's LDS addresses
+  // in slot 0.
+  uint32_t vr[NB][2];
+#pragma unroll
+  for (int db = 0; db < NB; db++)
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++) {
+      const int kr = 16 * kt + 4 * g + (r16 >> 2), col = 16 * db + 4 * (r16 & 3);
+      vr[db][kt] = (uint32_t)(uintptr_t)(lds_void_t*)(va + wave * C::VSLOT) +
+                   (kr * VCH + C::vchunk_lds(kr, col >> 3)) * 16 + (col & 7) * 2;
+    }
+
+  f32x4_t sc[SV][2];
+  unsigned short mk[MASK ? SV : 1][8];
+  using VV = u32x2_t[NB][2];
+  // Values of slot u, transposed (issued only: vwait before use).
+  auto vread = [&](int u, VV& vv) __attribute__((always_inline)) {
+#pragma unroll
+    for (int db = 0; db < NB; db++)
+#pragma unroll
+      for (int kt = 0; kt < 2; kt++) {
+        if constexpr (SV * C::ARR_U4 * 16 <= 65536)
+          vv[db][kt] = ds_read_tr_at(vr[db][kt], u * C::ARR_U4 * 16);
+        else
+          vv[db][kt] = ds_read_tr(vr[db][kt] + u * C::ARR_U4 * 16);
+      }
+  };
+  auto vwait = [&](VV& vv) __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int db = 0; db < NB; db++) asm volatile("" : "+v"(vv[db][0]), "+v"(vv[db][1]));
+  };
+  // Block i in register set u: which keys the column uses, its scores r, the
+  // mask's addends t, and the largest score (without a mask: unscaled).
+  struct Block {
+    float r[2][4], t[2][4], bm;
+    bool use[2][4];
+    uint32_t used;
+  };
+  auto gather = [&](auto full_tag, int i, int u) __attribute__((always_inline)) -> Block {
+    constexpr bool FULL = decltype(full_tag)::value;
+    const int key0 = (wave + kWaves * i) * kBlk + 4 * g;
+    Block k;
+    k.bm = -INFINITY;
+    k.used = 0;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        k.r[kt][e] = sc[u][kt][e];
+        k.use[kt][e] = FULL || key0 + 16 * kt + e < kend;
+        if constexpr (MASK) {
+          const float mv = (float)__builtin_bit_cast(T, mk[u][4 * kt + e]);
+          k.use[kt][e] = k.use[kt][e] && mv > -3.0e38f;
+          k.t[kt][e] = mv * kLog2e;
+          const float sv = k.r[kt][e] * p.ascale2 + k.t[kt][e];
+          k.bm = k.use[kt][e] ? fmaxf(k.bm, sv) : k.bm;
+          k.used |= k.use[kt][e] ? 1u << (4 * kt + e) : 0u;
+        } else {
+          k.t[kt][e] = 0.f;
+          k.bm = k.use[kt][e] ? fmaxf(k.bm, k.r[kt][e]) : k.bm;
+        }
+      }
+    return k;
+  };
+  // The block's probabilities from base m, packed, and their sum.
+  auto probs = [&](const Block& k, float& ps) __attribute__((always_inline)) -> uint4 {
+    float pv[2][4];
+    ps = 0.f;
+#pragma unroll
+    for (int kt = 0; kt < 2; kt++)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float a = MASK ? k.t[kt][e] - m : -m;
+        pv[kt][e] = k.use[kt][e]
+                        ? __builtin_amdgcn_exp2f(__builtin_fmaf(k.r[kt][e], p.ascale2, a)) : 0.f;
+        ps = kt + e == 0 ? pv[0][0] : ps + pv[kt][e];
+      }
+    ps = col_sum(ps);
+    return join(pack_p<T>(pv[0]), pack_p<T>(pv[1]));
+  };
+  // o += P . V; with a mask, values of keys that no column uses are zeroed
+  // (see sdpa_mfma_kernel).
+  auto product = [&](uint4 ph, uint32_t used, VV& vv) __attribute__((always_inline)) {
+    if constexpr (MASK) {
+      used |= __builtin_amdgcn_mov_dpp((int)used, 0x121, 0xF, 0xF, false);  // row_ror:1
+      used |= __builtin_amdgcn_mov_dpp((int)used, 0x122, 0xF, 0xF, false);  // row_ror:2
+      used |= __builtin_amdgcn_mov_dpp((int)used, 0x124, 0xF, 0xF, false);  // row_ror:4
+      used |= __builtin_amdgcn_mov_dpp((int)used, 0x128, 0xF, 0xF, false);  // row_ror:8
+      if (__builtin_amdgcn_ballot_w64(used != 0xFFu) != 0) {  // wave-uniform
+#pragma unroll
+        for (int kt = 0; kt < 2; kt++) {
+          uint32_t keep[4];
+#pragma unroll
+          for (int e = 0; e < 4; e++) keep[e] = (used >> (4 * kt + e)) & 1 ? 0xFFFFu : 0u;
+          const u32x2_t vm = {keep[0] | (keep[1] << 16), keep[2] | (keep[3] << 16)};
+#pragma unroll
+          for (int db = 0; db < NB; db++) vv[db][kt] &= vm;
+        }
+      }
+    }
+#pragma unroll
+    for (int db = 0; db < NB; db++)
+      o[db] = mma32(T(0), join(__builtin_bit_cast(uint2, vv[db][0]), __builtin_bit_cast(uint2, vv[db][1])),
+                    ph, o[db]);
+  };
+  auto moves = [&](float bm) __attribute__((always_inline)) -> bool {  // wave-uniform
+    return __builtin_amdgcn_ballot_w64((MASK ? bm : bm * p.ascale2) > m + 8.f) != 0;
+  };
+  auto step = [&](const Block& k, VV& vv) __attribute__((always_inline)) {
+    float f = 1.f;
+    if (moves(k.bm)) {
+      const float bm = MASK ? col_max(k.bm) : col_max(k.bm) * p.ascale2;
+      const float mn = bm > -INFINITY && bm > m + 8.f ? bm : m;
+      if (mn != m) {
+        f = __builtin_amdgcn_exp2f(m - mn);
+        if (f != 1.f) {
+#pragma unroll
+          for (int db = 0; db < NB; db++) o[db] = o[db] * f + 0.f;
+        }
+      }
+      m = mn;
+    }
+    float ps;
+    const uint4 ph = probs(k, ps);
+    l = __builtin_fmaf(l, f, ps);
+    product(ph, k.used, vv);
+  };
+  // Blocks i .. i + PB - 1, in register sets and slots u ..: where no base
+  // moves in any of them, they depend on each other through the sums l and o
+  // alone, and their softmaxes run side by side.
+  auto group = [&](auto full_tag, int i, int u) __attribute__((always_inline)) {
+    VV vv[PB];
+    Block k[PB];
+    float bm = -INFINITY;
+#pragma unroll
+    for (int j = 0; j < PB; j++) vread(u + j, vv[j]);
+#pragma unroll
+    for (int j = 0; j < PB; j++) {
+      k[j] = gather(full_tag, i + j, u + j);
+      bm = fmaxf(bm, k[j].bm);
+    }
+    if (PB > 1 && !moves(bm)) {
+      uint4 ph[PB];
+      float ps[PB];
+#pragma unroll
+      for (int j = 0; j < PB; j++) ph[j] = probs(k[j], ps[j]);
+#pragma unroll
+      for (int j = 0; j < PB; j++) l = __builtin_fmaf(l, 1.f, ps[j]);
+#pragma unroll
+      for (int j = 0; j < PB; j++) vwait(vv[j]);
+#pragma unroll
+      for (int j = 0; j < PB; j++) product(ph[j], k[j].used, vv[j]);
+    } else {
+#pragma unroll
+      for (int j = 0; j < PB; j++) vwait(vv[j]);
+#pragma unroll
+      for (int j = 0; j < PB; j++) step(k[j], vv[j]);
+    }
+  };
+  // The loads of the PB blocks that follow those in flight, into the sets and
+  // slots of the last group's (whose reads have returned); then group u has
+  // landed.
+  auto next = [&](int u) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < PB; j++) {
+      const int w = (u + SV - PB + j) % SV;
+      ld.sload(sc[w], mk[MASK ? w : 0]);
+      ld.vload(va + w * C::ARR_U4 + wave * C::VSLOT);
+    }
+    __builtin_amdgcn_s_waitcnt(wait_vm(VWAIT));
+  };
+#pragma unroll
+  for (int u = 0; u < SV - PB; u++) {
+    ld.sload(sc[u], mk[MASK ? u : 0]);
+    ld.vload(va + u * C::ARR_U4 + wave * C::VSLOT);
+  }
+  const int whole = MASK ? nit : nfit;  // blocks that whole groups may take
+  int i0 = 0;
+  for (; i0 + SV <= whole; i0 += SV) {
+#pragma unroll
+    for (int u = 0; u < SV; u += PB) {
+      next(u);
+      group(std::integral_constant<bool, !MASK>{}, i0 + u, u);
+    }
+  }
+  for (; i0 < nit; i0 += SV) {
+#pragma unroll
+    for (int u = 0; u < SV; u += PB) {
+      if (i0 + u >= nit) break;
+      next(u);
+#pragma unroll
+      for (int j = 0; j < PB; j++)
+        if (i0 + u + j < nit) {
+          VV vv;
+          vread(u + j, vv);
+          const Block k = gather(std::false_type{}, i0 + u + j, u + j);
+          vwait(vv);
+          step(k, vv);
+        }
+    }
+  }
+
+  // Merge, as sdpa_mfma_kernel: o of chain c in slot 0, (m, l) in slot 1.
+  uint4* const mrg = va;
+  float2* const ml = reinterpret_cast<float2*>(va + C::ARR_U4);
+  __builtin_amdgcn_s_waitcnt(kWaitAll);
+  asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+  for (int db = 0; db < NB; db++)
+    st16(mrg + (wave * NB + db) * 64 + lane, __builtin_bit_cast(uint4, o[db]));
+  ml[wave * 64 + lane] = make_float2(m, l);
+  __builtin_amdgcn_s_waitcnt(kWaitAll);
+  asm volatile("s_barrier" ::: "memory");
+  float mc[kWaves], lc[kWaves], ec[kWaves];
+  const float sk = p.sinks ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
+  float M = sk;
+#pragma unroll
+  for (int c = 0; c < kWaves; c++) {
+    const float2 v = ml[c * 64 + lane];
+    mc[c] = v.x;
+    lc[c] = v.y;
+    M = fmaxf(M, mc[c]);
+  }
+  float L = p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
+#pragma unroll
+  for (int c = 0; c < kWaves; c++) {
+    ec[c] = __builtin_amdgcn_exp2f(mc[c] - M);
+    L = __builtin_fmaf(lc[c], ec[c], L);
+  }
+  T* __restrict__ out = static_cast<T*>(p.out) + ((b * p.H + head) * p.qL + srow) * V + ws * C::DW;
+#pragma unroll
+  for (int k = 0; k < (NB + kWaves - 1) / kWaves; k++) {
+    const int db = wave + kWaves * k;
+    if (db >= NB) break;
+    f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < kWaves; c++) {
+      const f32x4_t oc = __builtin_bit_cast(f32x4_t, ld16(mrg + (c * NB + db) * 64 + lane));
+#pragma unroll
+      for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
+    }
+    O += 0.f;
+    unsigned short ob[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
+    if (colv)
+      *reinterpret_cast<uint2*>(out + 16 * db + 4 * g) =
+          make_uint2(ob[0] | ((uint32_t)ob[1] << 16), ob[2] | ((uint32_t)ob[3] << 16));
+  }
 }
 
 // f(integral_constant<I>) for I = I0 .. N - 1 while it returns true.
@@ -1230,13 +1475,12 @@ struct Shared {
   };
 };
 
-template <typename T, int D, int V, int NW, int GP, int NG, int SEG>
+template <typename T, int D, int V, int NW, int GP, int NG>
 __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
   using C = Shared<T, D, V, NW, GP, NG>;
   constexpr int NQ = C::NQ, NB = C::NB, CH = C::CH, VCH = C::VCH, LPW = C::LPW;
   constexpr int COLS = 16 * NW;  // columns per workgroup
   __shared__ uint4 ring[C::S * C::SLOT];
-
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -1477,84 +1721,23 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
     static_for<0, GP>(blockstep);
     return true;
   };
-  // SEG_WALK: the running state (R, S, Q) over the segments so far; Q in LDS
-  // (in registers it would not fit beside the 4 chains' state).
-  float R = -FLT_MAX, S = 0.f;
-  bool folded = false;
-  auto run_lds = []() __attribute__((always_inline)) -> uint4* {
-    if constexpr (SEG == SEG_WALK) {
-      __shared__ uint4 run[NW * NB * 64];
-      return run;
-    }
-    return nullptr;
-  };
-  static_assert(kSegBlk % (UG * GP) == 0, "segments end on a round of the loop");
-  if constexpr (SEG == SEG_WALK) {
-    // Every segment but the last: its blocks, then, for a wave whose columns
-    // see keys past it, its chains merge and fold.
-    for (int end = kSegBlk; end < nblk; end += kSegBlk) {
-      for (; q0 * GP < end; q0 += UG) static_for<0, UG>(group);
-      if (end < nvis_w) {
-        const bool sink = p.sinks && !folded;
-        const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
-        float M = sk;
-#pragma unroll
-        for (int c = 0; c < 4; c++) M = fmaxf(M, m[c]);
-        float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;
-        float ec[4];
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          ec[c] = __builtin_amdgcn_exp2f(m[c] - M);
-          L = __builtin_fmaf(l[c], ec[c], L);
-        }
-        const FoldW w = fold_stats(R, S, M, L);
-        uint4* const run = run_lds() + wave * NB * 64 + lane;
-#pragma unroll
-        for (int db = 0; db < NB; db++) {
-          f32x4_t O = f32x4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-          for (int c = 0; c < 4; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(o[c][db][e], ec[c], O[e]);
-          f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
-          if (folded) Q = __builtin_bit_cast(f32x4_t, ld16(run + db * 64));  // wave-uniform
-          fold_out(Q, O, w);
-          st16(run + db * 64, __builtin_bit_cast(uint4, Q));
-        }
-        folded = true;
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          m[c] = -FLT_MAX;
-          l[c] = 0.f;
-#pragma unroll
-          for (int i = 0; i < NB; i++) o[c][i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-        }
-      }
-    }
-  }
   for (; q0 * GP < nblk; q0 += UG) static_for<0, UG>(group);
   // The loads issued past the last block (they read nothing but still write
   // their slots) complete before the workgroup's LDS is released.
   __builtin_amdgcn_s_waitcnt(kWaitAll);
 
-  // Merge the 4 chains in order, in registers (the sink first, in the first
-  // segment: -FLT_MAX without one).
-  const bool sink = SEG == SEG_ONE ? p.sinks != nullptr : p.sinks && !folded;
-  const float sk = sink ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
+  // Merge the 4 chains in order, in registers (the sink first: -FLT_MAX
+  // without one).
+  const float sk = p.sinks ? (float)static_cast<const T*>(p.sinks)[head] * kLog2e : -FLT_MAX;
   float M = sk;
 #pragma unroll
   for (int c = 0; c < 4; c++) M = fmaxf(M, m[c]);
-  float L = sink ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
+  float L = p.sinks ? __builtin_amdgcn_exp2f(sk - M) : 0.f;  // the sink's l = 1
   float ec[4];
 #pragma unroll
   for (int c = 0; c < 4; c++) {
     ec[c] = __builtin_amdgcn_exp2f(m[c] - M);
     L = __builtin_fmaf(l[c], ec[c], L);
-  }
-  FoldW w = {0.f, 0.f};
-  if constexpr (SEG == SEG_WALK) {
-    w = fold_stats(R, S, M, L);
-    L = S;
   }
   T* __restrict__ out = static_cast<T*>(p.out) + ((b * p.H + head) * p.qL + srow) * V;
 #pragma unroll
@@ -1564,14 +1747,7 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
     for (int c = 0; c < 4; c++)
 #pragma unroll
       for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(o[c][db][e], ec[c], O[e]);
-    if constexpr (SEG == SEG_WALK) {
-      f32x4_t Q = f32x4_t{0.f, 0.f, 0.f, 0.f};
-      if (folded) Q = __builtin_bit_cast(f32x4_t, ld16(run_lds() + (wave * NB + db) * 64 + lane));
-      fold_out(Q, O, w);
-      O = Q;
-    } else {
-      O += 0.f;
-    }
+    O += 0.f;
     unsigned short ob[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
@@ -1594,63 +1770,90 @@ constexpr int sdpa_loader_slots(int D, int V, int WS) {
 // through LDS by contiguous loads (sdpa_loader_slots). Wide heads (D or V above
 // 128) load no keys ahead. Keys one block ahead and values in two slots
 // otherwise: deeper prefetch measured no faster.
-template <typename T, int D, int V, bool MASK, int SHAPE, int SEG>
+template <typename T, int D, int V, bool MASK, int SHAPE>
 constexpr SdpaKernelFn mfma_kernel() {
   constexpr int MK = MASK ? 1 : 0;
   constexpr int PK = sdpa_wide(D, V) ? 0 : 1;
   constexpr int WS = sdpa_shape_splits(V, SHAPE);
   if constexpr (SHAPE == SDPA_SHARED) {
-    if constexpr (sdpa_shared_dims(D, V) && !MASK && SEG != SEG_SPLIT)
-      return sdpa_shared_kernel<T, D, V, sdpa_shared_waves(D, V), 2, 2, SEG>;
+    if constexpr (sdpa_shared_dims(D, V) && !MASK)
+      return sdpa_shared_kernel<T, D, V, sdpa_shared_waves(D, V), 2, 2>;
     else
       return nullptr;
   } else if constexpr (SHAPE == SDPA_ROWS) {
-    constexpr int CT = sdpa_rows_tiles(D, V);
-    if constexpr (CT == 2 && SEG == SEG_WALK)
-      return sdpa_mfma_kernel2<T, D, V, CT, MASK ? 0 : PK, 2, WS, MASK ? 2 : 0, false, 0, SEG>;
-    else
-      return sdpa_mfma_kernel<T, D, V, CT, MASK ? 0 : PK, 2, WS, MASK ? 2 : 0, false, 0, SEG>;
+    return sdpa_mfma_kernel<T, D, V, sdpa_rows_tiles(D, V), MASK ? 0 : PK, 2, WS, MASK ? 2 : 0,
+                            false, 0>;
   } else if constexpr (SHAPE == SDPA_TILE) {
-    return sdpa_mfma_kernel<T, D, V, 1, PK, 2, WS, MK, false, 0, SEG>;
+    return sdpa_mfma_kernel<T, D, V, 1, PK, 2, WS, MK, false, 0>;
   } else {
     // Keys in LDS with loader waves (sdpa_loaders: the host launches 8 waves).
     constexpr bool KLS = sdpa_loaders(D, V, SHAPE, MASK);
     return sdpa_mfma_kernel<T, D, V, 1, KLS ? 0 : PK, KLS ? sdpa_loader_slots(D, V, WS) : 2, WS, MK, KLS,
-                            KLS ? kWaves : 0, SEG>;
+                            KLS ? kWaves : 0>;
   }
 }
 
+// Value slots of a SDPA_SCORED kernel, and blocks a group takes side by side:
+// as many as LDS (64 KB) and the count of loads in flight (63) allow.
+constexpr int sdpa_scored_slots(int DW, bool MASK) {
+  return DW <= 16 && !MASK ? 12 : DW <= 32 ? 8 : DW <= 64 ? 4 : 2;
+}
+constexpr int sdpa_scored_group(int DW) { return DW <= 32 ? 4 : DW <= 64 ? 2 : 1; }
+
+// SDPA_SCORES (shape: column tiles per workgroup) and SDPA_SCORED kernels.
+template <typename T, int D>
+SdpaKernelFn mfma_scores(int tiles) {
+  if constexpr (D <= 256) {
+    if (tiles == 2) return sdpa_scores_kernel<T, D, 2>;
+  }
+  return tiles == 1 ? sdpa_scores_kernel<T, D, 1> : nullptr;
+}
 template <typename T, int D, int V, bool MASK, int SHAPE>
-SdpaKernelFn mfma_kernel_seg(int seg) {
-  switch (seg) {
-    case SEG_ONE: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_ONE>();
-    case SEG_WALK: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_WALK>();
-    case SEG_SPLIT: return mfma_kernel<T, D, V, MASK, SHAPE, SEG_SPLIT>();
+constexpr SdpaKernelFn mfma_scored() {
+  constexpr int WS = sdpa_shape_splits(V, SHAPE);
+  constexpr int SV = sdpa_scored_slots(V / WS, MASK), PB = sdpa_scored_group(V / WS);
+  return sdpa_scored_kernel<T, V, SV, PB, WS, MASK>;
+}
+template <typename T, int D, int V, bool MASK>
+SdpaKernelFn mfma_scored_shape(int shape) {
+  switch (shape) {
+    case SDPA_TILE: return mfma_scored<T, D, V, MASK, SDPA_TILE>();
+    case SDPA_SPLIT2: return mfma_scored<T, D, V, MASK, SDPA_SPLIT2>();
+    case SDPA_SPLIT4: return mfma_scored<T, D, V, MASK, SDPA_SPLIT4>();
+    case SDPA_SPLIT8: return mfma_scored<T, D, V, MASK, SDPA_SPLIT8>();
   }
   return nullptr;
 }
 
 template <typename T, int D, int V, bool MASK>
-SdpaKernelFn mfma_kernel_shape(int shape, int seg) {
+SdpaKernelFn mfma_kernel_shape(int shape) {
   switch (shape) {
-    case SDPA_ROWS: return mfma_kernel_seg<T, D, V, MASK, SDPA_ROWS>(seg);
-    case SDPA_TILE: return mfma_kernel_seg<T, D, V, MASK, SDPA_TILE>(seg);
-    case SDPA_SPLIT2: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT2>(seg);
-    case SDPA_SPLIT4: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT4>(seg);
-    case SDPA_SPLIT8: return mfma_kernel_seg<T, D, V, MASK, SDPA_SPLIT8>(seg);
-    case SDPA_SHARED: return mfma_kernel_seg<T, D, V, MASK, SDPA_SHARED>(seg);
+    case SDPA_ROWS: return mfma_kernel<T, D, V, MASK, SDPA_ROWS>();
+    case SDPA_TILE: return mfma_kernel<T, D, V, MASK, SDPA_TILE>();
+    case SDPA_SPLIT2: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT2>();
+    case SDPA_SPLIT4: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT4>();
+    case SDPA_SPLIT8: return mfma_kernel<T, D, V, MASK, SDPA_SPLIT8>();
+    case SDPA_SHARED: return mfma_kernel<T, D, V, MASK, SDPA_SHARED>();
+  }
+  return nullptr;
+}
+
+template <typename T, int D, int V>
+SdpaKernelFn mfma_kernel_stage(bool mask, int shape, int stage) {
+  switch (stage) {
+    case SDPA_WHOLE:
+      return mask ? mfma_kernel_shape<T, D, V, true>(shape) : mfma_kernel_shape<T, D, V, false>(shape);
+    case SDPA_SCORES: return mfma_scores<T, D>(shape);
+    case SDPA_SCORED:
+      return mask ? mfma_scored_shape<T, D, V, true>(shape) : mfma_scored_shape<T, D, V, false>(shape);
   }
   return nullptr;
 }
 
 template <int D, int V>
-SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape, int seg) {
-  if (dtype == BI_BF16)
-    return mask ? mfma_kernel_shape<__bf16, D, V, true>(shape, seg)
-                : mfma_kernel_shape<__bf16, D, V, false>(shape, seg);
-  if (dtype == BI_F16)
-    return mask ? mfma_kernel_shape<_Float16, D, V, true>(shape, seg)
-                : mfma_kernel_shape<_Float16, D, V, false>(shape, seg);
+SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape, int stage) {
+  if (dtype == BI_BF16) return mfma_kernel_stage<__bf16, D, V>(mask, shape, stage);
+  if (dtype == BI_F16) return mfma_kernel_stage<_Float16, D, V>(mask, shape, stage);
   return nullptr;
 }
 
@@ -1658,7 +1861,7 @@ SdpaKernelFn mfma_kernel_for(int dtype, bool mask, int shape, int seg) {
 
 // Defines the lookup of one head-dim pair's kernels (declared in
 // bi_sdpa_args.h); each instantiation unit expands it once.
-#define BI_SDPA_MFMA_DEFINE(D, V)                                                        \
-  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int seg) {  \
-    return mfma_kernel_for<D, V>(dtype, mask, shape, seg);                               \
+#define BI_SDPA_MFMA_DEFINE(D, V)                                                          \
+  SdpaKernelFn sdpa_mfma_kernel_d##D##_v##V(int dtype, bool mask, int shape, int stage) {  \
+    return mfma_kernel_for<D, V>(dtype, mask, shape, stage);                               \
   }

@@ -5,13 +5,14 @@ normalisation, validation, sinks, launch) on top of the HIP kernels in
 csrc/ (bi_sdpa.hip: fp32 on the vector ALUs; bi_sdpa_mfma_kernel.h: bf16 and
 f16 on matrix cores), reached through the C ABI ``bi_sdpa`` (include/bi.h).
 
-fp32 splits a query row's reduction over the keys into 32 partial online
-softmaxes by key index (key i belongs to partial i mod 32) in one workgroup;
-bf16/f16 into segments of 2048 keys at fixed positions, each into 4 chains of
-32-key blocks (block b belongs to chain b mod 4), in one workgroup or, for
-grids that would leave the GPU idle, one per segment. The partials are combined
-in a fixed order. Nothing in that order depends on the number of query rows,
-the batch, or how far the key sequence extends past the keys a row can see.
+One workgroup owns the entire reduction over the keys for each of its query
+rows. fp32 splits it into 32 partial online softmaxes by key index (key i
+belongs to partial i mod 32); bf16/f16 into 4 chains of 32-key blocks (block b
+belongs to chain b mod 4); the partials are combined in a fixed order. Nothing
+in that order depends on the number of query rows, the batch, or how far the
+key sequence extends past the keys a row can see. Where the grid would leave
+the GPU idle, bf16/f16 scores, which depend on nothing but their query and key,
+come from a kernel of their own through a workspace; the bits are the same.
 """
 
 import ctypes
@@ -83,6 +84,9 @@ def _kernel_view(t):
 
 _NO_MASK_STRIDES = _lib.i64_array((0, 0, 0))
 _I64x9 = ctypes.c_int64 * 9
+# Keys times head dim below which bi_sdpa_workspace always answers 0
+# (csrc/bi_sdpa.hip pick_scored): short calls are not worth asking for.
+_SCORES_MIN = 192 * 1024
 
 
 def _sdpa(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks):
@@ -101,8 +105,8 @@ def _sdpa(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks):
 def _sdpa_eager(q, k, v, scale, mask_mode, mask, mstrides, causal_offset, sinks, shape=None,
                 split=False):
     """The launch; `shape` forces a launch shape (bi_sdpa_with_shape,
-    include/bi_testing.h) instead of the one bi_sdpa picks, `split` one segment
-    of the keys per workgroup in it (bi_sdpa_split_with_shape)."""
+    include/bi_testing.h) instead of the one bi_sdpa picks, `split` the scores
+    by a kernel of their own (bi_sdpa_split_with_shape)."""
     B, H, qL, D = q.shape
     _, Hkv, N, _ = k.shape
     V = v.shape[-1]
@@ -136,8 +140,9 @@ def _launch(L, args, shape, split, q, stream):
         return L.bi_sdpa_with_shape(*args, int(shape), stream)
     need = 0
     if split:
-        need = B * H * qL * -(-N // _lib.SDPA_SEGMENT) * (V + 2) * 4
-    elif N > _lib.SDPA_SEGMENT:
+        ncol = H // Hkv * qL
+        need = B * Hkv * -(-ncol // 16) * -(-N // 32) * 32 * min(16, ncol) * 4
+    elif N * D >= _SCORES_MIN and args[18] != _lib.F32:
         need = L.bi_sdpa_workspace(B, H, Hkv, qL, N, D, V, args[18], args[16])
     if not need:
         return L.bi_sdpa(*args, stream)

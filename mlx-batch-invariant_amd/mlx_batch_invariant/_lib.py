@@ -74,7 +74,6 @@ SIGNATURES = {
 # Attention launch shapes (include/bi_testing.h): bf16 / f16 on matrix cores.
 SDPA_ROWS, SDPA_TILE, SDPA_SPLIT2, SDPA_SPLIT4, SDPA_SPLIT8, SDPA_SHARED = 0, 1, 2, 3, 4, 5
 SDPA_NUM_SHAPES = 6
-SDPA_SEGMENT = 2048  # keys per segment of the bf16/f16 kernels (bi_sdpa_args.h kSegKeys)
 
 ABI_VERSION = 1
 

@@ -26,6 +26,7 @@ import numpy as np
 import pytest
 import torch
 
+import mlx_batch_invariant as bi
 from mlx_batch_invariant import _attention, _lib
 from oracle import sdpa as osdpa
 
@@ -482,11 +483,11 @@ def test_fp32_head_grouping_prefill(cuda):
 @pytest.mark.parametrize("D,V", [(128, 128), (64, 64), (256, 256), (576, 512)])
 @pytest.mark.parametrize("N", [2047, 2049, 4096, 6200])
 def test_segments_give_the_same_bits_in_one_workgroup_or_each_in_its_own(cuda, D, V, N):
-    """bf16 / f16: past one segment of keys, every launch shape that walks all
-    segments and every one that takes one segment per workgroup, with a second
-    kernel folding them, gives the same bits: without a mask, causal with
-    sinks, and with an additive mask that hides the whole first or last
-    segment from some rows; rows against float64."""
+    """bf16 / f16: every launch shape that computes its scores and every one that
+    reads them from the scores kernel ("split") gives the same bits at contexts
+    around 2048 keys and multiples of it: without a mask, causal with sinks, and
+    with an additive mask that hides the first 2048 keys or the last 2048 from
+    some rows; rows against float64."""
     H, Hkv, qL, B = 8, 2, 5, 2
     for dname, dtype in (("float16", torch.float16), ("bfloat16", torch.bfloat16)):
         q = rn((B, H, qL, D), dtype, 71, device=cuda)
@@ -558,12 +559,12 @@ def _underflowing(B, H, Hkv, qL, N, D, dtype, device, low_block, rest):
 
 @pytest.mark.parametrize("dname,dtype", LOW)
 def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
-    """A negative result below the fp32 range is +0.0 in every launch shape,
-    with one segment of keys or with more behind it (hidden by the mask, or by
-    the causal bound), walked or one per workgroup: its sign does not depend
-    on the context's length or on the route."""
+    """A negative result below the fp32 range is +0.0 in every launch shape, for
+    contexts of any length (the rest hidden by the mask, or by the causal
+    bound) and with the scores from either kernel: its sign does not depend on
+    the context's length or on the route."""
     B, H, Hkv, qL, D = 1, 8, 2, 5, 128
-    for low_block in (3, 2, 67):  # the last chain, an earlier one, the second segment
+    for low_block in (3, 2, 67):  # the last chain, an earlier one, far along the keys
         for N in (2048, 2112, 4300, 8192):
             if 32 * low_block >= N:
                 continue
@@ -587,3 +588,161 @@ def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
                     off = 2000  # rows 0..63 see keys up to 2000..2063
                 y = _attention._sdpa_eager(q, k, v, 1.0, mode, m, ms, off, None, shape=shape)
                 assert not bits(y).any(), (dname, N, spec, shape)
+
+
+def _ws_bytes(B, H, Hkv, qL, N):
+    c = H // Hkv * qL
+    return B * Hkv * -(-c // 16) * -(-N // 32) * 128 * min(c, 16)
+
+
+@pytest.mark.parametrize("D,V", PAIRS)
+def test_scores_kernel_gives_the_same_bits(cuda, D, V):
+    """The scores route (raw scores by a kernel of their own, the rest reading
+    them) gives the one-kernel shapes' bits: key counts below, at and past a
+    block, a chain's round and a group of blocks; fewer columns than a tile,
+    a last tile cut short, an odd number of tiles; more query rows than keys;
+    additive and boolean masks (-inf, the type's lowest value, an infinite
+    score), sinks, a negative scale, bases that move in every block, and NaNs
+    in the keys and values no row sees."""
+    L = _lib.lib()
+    cases = [(1, 8, 2, 1, 1), (2, 8, 2, 1, 31), (1, 4, 4, 3, 33), (1, 8, 2, 5, 129),
+             (1, 6, 2, 11, 257), (2, 8, 1, 5, 1000), (1, 2, 2, 40, 1100), (1, 8, 2, 9, 4),
+             (1, 8, 8, 1, 2100)]
+    for dname, dtype in LOW:
+        low = torch.finfo(dtype).min
+        for n, (B, H, Hkv, qL, N) in enumerate(cases):
+            q = rn((B, H, qL, D), dtype, 500 + n, device=cuda)
+            cache_k = rn((B, Hkv, N + 40, D), dtype, 520 + n, device=cuda)
+            cache_v = rn((B, Hkv, N + 40, V), dtype, 540 + n, device=cuda)
+            cache_k[:, :, N:] = float("nan")
+            cache_v[:, :, N:] = float("nan")
+            k, v = cache_k[:, :, :N], cache_v[:, :, :N]
+            sinks = rn((H,), dtype, 560, device=cuda)
+            add, keep = _masks(B, qL, N, dtype, cuda, 580 + n)
+            add[:, :, :, ::7] = low
+            if N > 3:
+                add[0, 0, -1, 2] = float("inf")
+            rising = k.clone()
+            rising[..., 0] = torch.arange(N, device=cuda, dtype=torch.float32).to(dtype) / 2
+            hidden_k, hidden_v = cache_k.clone(), cache_v.clone()
+            hidden_k[:, :, max(1, N - 20):] = float("nan")
+            hidden_v[:, :, max(1, N - 20):] = float("nan")
+            seen = torch.zeros(1, 1, 1, N, dtype=torch.bool, device=cuda)
+            seen[..., :max(1, N - 20)] = True
+            for label, kk, vv, spec, sk, scale in (
+                    ("none", k, v, None, None, D ** -0.5), ("end", k, v, "end", sinks, D ** -0.5),
+                    ("start", k, v, "start", None, -0.3), ("additive", k, v, add, sinks, D ** -0.5),
+                    ("bool", k, v, keep, None, D ** -0.5), ("rising", rising, v, "end", None, 0.2),
+                    ("hidden", hidden_k[:, :, :N], hidden_v[:, :, :N], seen, None, D ** -0.5)):
+                mode, m, ms, off = _mask_mode(spec, q, kk)
+                ref = bits(_attention._sdpa_eager(q, kk, vv, scale, mode, m, ms, off, sk,
+                                                  shape=_lib.SDPA_TILE))
+                for shape in (_lib.SDPA_TILE, _lib.SDPA_SPLIT2, _lib.SDPA_SPLIT4, _lib.SDPA_SPLIT8):
+                    y = _attention._sdpa_eager(q, kk, vv, scale, mode, m, ms, off, sk, shape=shape,
+                                               split=True)
+                    case = "%s D=%d V=%d %s %s shape %d" % (dname, D, V, cases[n], label, shape)
+                    if label in ("none", "hidden"):
+                        assert torch.isfinite(y).all(), case
+                    d = int((bits(y) != ref).sum())
+                    assert d == 0, "%s: %d differ" % (case, d)
+    assert L.bi_sdpa_workspace(1, 8, 2, 1, 1, D, V, _lib.BF16, 0) == 0
+
+
+def _scores_problem(cuda, dtype=torch.bfloat16, B=1, qL=1, N=8192, seed=600):
+    q = rn((B, 32, qL, 128), dtype, seed, device=cuda)
+    k = rn((B, 8, N, 128), dtype, seed + 1, device=cuda)
+    v = rn((B, 8, N, 128), dtype, seed + 2, device=cuda)
+    need = _lib.lib().bi_sdpa_workspace(B, 32, 8, qL, N, 128, 128, _lib.DTYPE_CODES[dtype], 0)
+    return q, k, v, need
+
+
+def test_workspace_of_any_size_gives_the_same_bits(cuda):
+    """bi_sdpa_ws without a workspace, with one byte too few and with exactly
+    bi_sdpa_workspace's gives bi_sdpa's bits; exactly that many bytes are
+    written, and a misaligned buffer is refused."""
+    L = _lib.lib()
+    for dname, dtype in LOW:
+        q, k, v, need = _scores_problem(cuda, dtype)
+        assert need == _ws_bytes(1, 32, 8, 1, 8192)
+        want = run(q, k, v, None, shape=_lib.SDPA_TILE)
+        buf = torch.full((need + 4096,), 171, dtype=torch.uint8, device=cuda)
+        strides = _lib.i64_array((32 * 128, 128, 128) + 2 * (8 * 8192 * 128, 8192 * 128, 128))
+
+        def call(ptr, size):
+            out = torch.full_like(want, float("nan"))
+            rc = L.bi_sdpa_ws(q.data_ptr(), k.data_ptr(), v.data_ptr(), None, None, None,
+                              out.data_ptr(), 1, 32, 8, 1, 8192, 128, 128, strides,
+                              1.0 / math.sqrt(128), _lib.MASK_NONE, 0, _lib.DTYPE_CODES[dtype], ptr, size,
+                              torch.cuda.current_stream().cuda_stream)
+            return rc, out
+
+        for ptr, size in ((None, 0), (None, need), (buf.data_ptr(), need - 1)):
+            rc, out = call(ptr, size)
+            assert rc == _lib.OK and ndiff(out, want) == 0, (dname, size)
+            assert bool((buf == 171).all())
+        rc, out = call(buf.data_ptr(), need)
+        assert rc == _lib.OK and ndiff(out, want) == 0, dname
+        assert bool((buf[need:] == 171).all()) and not bool((buf[:need] == 171).all())
+        assert call(buf.data_ptr() + 8, need)[0] == _lib.EINVAL
+
+
+def test_workspace_route_in_a_graph_and_on_two_streams(cuda):
+    """The route with a workspace, captured and replayed with other attention
+    calls and allocations between the replays, and run on two streams at once
+    with different inputs: every result has the eager call's bits."""
+    q, k, v, need = _scores_problem(cuda)
+    assert need > 0
+    eager = bi.scaled_dot_product_attention(q, k, v).clone()
+    assert ndiff(eager, run(q, k, v, None, shape=_lib.SDPA_TILE)) == 0
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        bi.scaled_dot_product_attention(q, k, v)
+    torch.cuda.current_stream().wait_stream(s)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = bi.scaled_dot_product_attention(q, k, v)
+    q2, k2, v2, _ = _scores_problem(cuda, seed=620)
+    eager2 = bi.scaled_dot_product_attention(q2, k2, v2).clone()
+    for rep in range(4):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert ndiff(y, eager) == 0, rep
+        junk = torch.full((need,), 255, dtype=torch.uint8, device=cuda)
+        assert ndiff(bi.scaled_dot_product_attention(q2, k2, v2), eager2) == 0, rep
+        del junk
+        torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    for st in streams:
+        st.wait_stream(torch.cuda.current_stream())
+    outs = [[], []]
+    for rep in range(8):
+        for i, (st, a) in enumerate(zip(streams, ((q, k, v), (q2, k2, v2)))):
+            with torch.cuda.stream(st):
+                outs[i].append(bi.scaled_dot_product_attention(*a))
+    torch.cuda.synchronize()
+    for i, want in enumerate((eager, eager2)):
+        for rep, got in enumerate(outs[i]):
+            assert ndiff(got, want) == 0, (i, rep)
+
+
+def test_picked_route_is_invariant_along_the_batch_and_query_rows(cuda):
+    """Problems that take the scores route and problems that do not, as
+    bi_sdpa_workspace says, give a row the same bits: batch 1 and 16, query
+    rows 1 and 64 of a causal chunk, with and without an array mask."""
+    L = _lib.lib()
+    for dname, dtype in LOW:
+        for D, N in ((128, 6000), (64, 9000), (256, 2500)):
+            q = rn((16, 16, 64, D), dtype, 700, device=cuda)
+            k = rn((16, 4, N, D), dtype, 701, device=cuda)
+            v = rn((16, 4, N, D), dtype, 702, device=cuda)
+            code = _lib.DTYPE_CODES[dtype]
+            assert L.bi_sdpa_workspace(1, 16, 4, 1, N, D, D, code, 0) > 0
+            assert L.bi_sdpa_workspace(16, 16, 4, 64, N, D, D, code, 1) == 0
+            full = bi.scaled_dot_product_attention(q, k, v, mask="causal")
+            one = bi.scaled_dot_product_attention(q[3:4, :, 63:], k[3:4], v[3:4])
+            assert ndiff(one[0, :, 0], full[3, :, 63].contiguous()) == 0, (dname, D)
+            zeros = torch.zeros(1, 1, 1, N, dtype=dtype, device=cuda)
+            one = bi.scaled_dot_product_attention(q[3:4, :, 63:], k[3:4], v[3:4], mask=zeros)
+            assert ndiff(one[0, :, 0], full[3, :, 63].contiguous()) == 0, (dname, D)
