@@ -43,8 +43,9 @@
 //     ahead of the chains: M = max of the sink's and the chains' m;
 //     L = exp2(sink2 - M) (0 without a sink), O = +0.0; then for
 //     c = 0, 1, 2, 3 in order, e_c = exp2(m_c - M), L = fma(l_c, e_c, L) and
-//     O = fma(o_c, e_c, O); O = O + 0.0 (a product that underflows from below
-//     leaves -0.0); out = L == 0 ? O : O / L, one rounding to T.
+//     O = fma(o_c, e_c, O); out = L == 0 ? O : O / L, one rounding to T.
+//     All four chains enter whatever N is, so how long the context is decides
+//     not even the sign of a result that underflows.
 //     (Seeding a chain's base with the sink, as the reference seeds its
 //     simdgroup 0, would put a large sink's p below f16's range.)
 // Every column, whatever workgroup or lane it lands in, however many rows or
@@ -878,7 +879,6 @@ __global__ void __launch_bounds__(kThreads + 64 * LW) sdpa_mfma_kernel(SdpaArgs 
 #pragma unroll
         for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
       }
-      O += 0.f;
       unsigned short ob[4];
 #pragma unroll
       for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
@@ -1347,7 +1347,6 @@ __global__ void __launch_bounds__(kThreads) sdpa_scored_kernel(SdpaArgs p) {
 #pragma unroll
       for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(oc[e], ec[c], O[e]);
     }
-    O += 0.f;
     unsigned short ob[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));
@@ -1747,7 +1746,6 @@ __global__ void __launch_bounds__(64 * NW) sdpa_shared_kernel(SdpaArgs p) {
     for (int c = 0; c < 4; c++)
 #pragma unroll
       for (int e = 0; e < 4; e++) O[e] = __builtin_fmaf(o[c][db][e], ec[c], O[e]);
-    O += 0.f;
     unsigned short ob[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) ob[e] = tbits((T)(L == 0.f ? O[e] : O[e] / L));

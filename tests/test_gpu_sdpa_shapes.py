@@ -558,12 +558,12 @@ def _underflowing(B, H, Hkv, qL, N, D, dtype, device, low_block, rest):
 
 
 @pytest.mark.parametrize("dname,dtype", LOW)
-def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
-    """A negative result below the fp32 range is +0.0 in every launch shape, for
-    contexts of any length (the rest hidden by the mask, or by the causal
-    bound) and with the scores from either kernel: its sign does not depend on
-    the context's length or on the route."""
+def test_underflow_gives_the_same_zero_whatever_the_context(cuda, dname, dtype):
+    """A negative result below the fp32 range is a zero of the same sign in every
+    launch shape, for contexts of any length (the rest hidden by the mask, or
+    by the causal bound) and with the scores from either kernel."""
     B, H, Hkv, qL, D = 1, 8, 2, 5, 128
+    zero = {}
     for low_block in (3, 2, 67):  # the last chain, an earlier one, far along the keys
         for N in (2048, 2112, 4300, 8192):
             if 32 * low_block >= N:
@@ -576,7 +576,9 @@ def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
                     mode, m, ms, off = _mask_mode(keep, q, k)
                     y = _attention._sdpa_eager(q, k, v, 1.0, mode, m, ms, off, None, shape=shape,
                                                split=split)
-                    assert not bits(y).any(), (dname, low_block, N, shape, split)
+                    assert bool((y == 0).all()), (dname, low_block, N, shape, split)
+                    zero.setdefault(low_block, set()).update(bits(y).ravel().tolist())
+                    assert len(zero[low_block]) == 1, (dname, low_block, N, shape, split)
     # Without a mask: the other keys score far below both (by 400), causal rows
     # of the shared shape among them.
     for N in (2048, 4300):
@@ -587,7 +589,9 @@ def test_underflow_gives_plus_zero_whatever_the_context(cuda, dname, dtype):
                 if spec:
                     off = 2000  # rows 0..63 see keys up to 2000..2063
                 y = _attention._sdpa_eager(q, k, v, 1.0, mode, m, ms, off, None, shape=shape)
-                assert not bits(y).any(), (dname, N, spec, shape)
+                assert bool((y == 0).all()), (dname, N, spec, shape)
+                zero.setdefault("far", set()).update(bits(y).ravel().tolist())
+                assert len(zero["far"]) == 1, (dname, N, spec, shape)
 
 
 def _ws_bytes(B, H, Hkv, qL, N):
