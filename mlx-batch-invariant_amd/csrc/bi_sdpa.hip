@@ -490,7 +490,7 @@ bool scored_fits(int64_t N, int64_t vs2, int esz) {
 // more (8 sequences, D = 128: 41 and 50 us).
 // Both times, in microseconds, by least squares over a grid of H/Hkv = 32/8,
 // 8/8, 16/2, seven head-dim pairs, B = 1..16, 1..32 query rows, N = 512..16384
-// with and without an array mask (1470 problems, everything cached: from HBM
+// with and without an array mask (1669 problems, everything cached: from HBM
 // the route gains more); at 0.8 of the whole's estimate it was faster in every
 // one it took, and took nine tenths of those where it gains a tenth.
 int pick_scored(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_t D, int64_t V,
@@ -509,16 +509,19 @@ int pick_scored(int64_t B, int64_t H, int64_t Hkv, int64_t qL, int64_t N, int64_
   const float c = 1.f / (float)cus, d = (float)D, dw = (float)(V / sdpa_shape_splits(V, shape));
   const float t = (float)tiles * c, wgs = t * (float)sdpa_shape_splits(V, shape);
   const float hbm = (float)streams * c;  // streams per compute unit
-  const float scored = (am ? 6.68f + 0.0282f * dw : 2.18f + 0.0115f * dw) + 0.1245f * d * hbm +
-                       0.1227f * wgs * dw + 0.1555f * t * (float)(ncol < 16 ? ncol : 16) +
-                       (D > 256 ? 5.1f : 0.f);
+  // Mask rows that a tile's columns read: its query rows.
+  const int64_t G = H / Hkv, tr = G < 16 ? 16 / G : 1;
+  const float mr = (float)(qL < tr ? qL : tr);
+  const float scored = (am ? 5.35f + 0.0259f * dw + 0.684f * mr : 2.05f + 0.0189f * dw) +
+                       0.137f * d * hbm + 0.1195f * wgs * dw +
+                       0.0462f * t * (float)(ncol < 16 ? ncol : 16) + (D > 256 ? 4.69f : 0.f);
   const float vw = (float)V / (float)sdpa_shape_splits(V, walk);
-  const float whole = (am                                ? 2.48f + 0.1222f * d + 0.0112f * vw
-                       : sdpa_loaders(D, V, walk, false) ? 0.0441f * d + 0.0318f * t * (float)(D + V)
-                                                         : 0.1112f * d + 0.0044f * t * (float)(D + V)) +
-                      0.0337f * (float)(D + V) * hbm;
+  const float whole = (am                                ? 1.24f + 0.1193f * d + 0.0166f * vw + 0.527f * mr
+                       : sdpa_loaders(D, V, walk, false) ? 0.0432f * d + 0.0318f * t * (float)(D + V)
+                                                         : 0.1112f * d + 0.0029f * t * (float)(D + V)) +
+                      0.0364f * (float)(D + V) * hbm;
   const float seg = (float)N / 2048.f;
-  return 8.1f + scored * seg < 0.8f * (3.73f + whole * seg) ? shape : -1;
+  return 8.11f + scored * seg < 0.8f * (3.75f + whole * seg) ? shape : -1;
 }
 
 // Validates, packs the arguments and launches shape `shape` (-1: the shape
