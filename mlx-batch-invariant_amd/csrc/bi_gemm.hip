@@ -119,8 +119,13 @@ int pick_geometry(int64_t M, int64_t N, int64_t K, int dtype, int trans_b) {
   // tiles are the ones where they fit one round and 64 x 64 ones take two (K =
   // 11008, N = 4096, M = 300: 56.9 against 67.1 us, (K, N) 61.0 against 68.1;
   // N = K = 2048, M = 1024: 13.5 against 15.6) and their 128 rows of A fit a
-  // buffer resource.
-  const bool panel = K < (int64_t)1 << 23;
+  // buffer resource. On (N, K) weights whose rows lie a multiple of 4 KB apart
+  // they take whole row tiles only: with weights from HBM, K = 4096, a last
+  // tile cut short costs more than the second round (M = 1200, N = 1024: 33.0
+  // against 30.1 us; M = 257, N = 4096: 32.5 and 30.7; M = 512, N = 4096: 34.4
+  // and 36.1; K = 11008 gains at every M).
+  const bool panel = K < (int64_t)1 << 23 &&
+                     !(trans_b && K >= 4096 && K % 2048 == 0 && M % 128);
   struct Cand { int g, bm, bn, w; };
   const Cand kCands[] = {{2, 64, 64, 129},
                          {3, 128, 128, 136},

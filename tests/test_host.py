@@ -144,13 +144,27 @@ def test_quantized_footprint_by_group_size():
     assert L.bi_qgemm_pick_group_geometry(1, 4096, 4096, 48, 4) == _lib.EINVAL
 
 
+def test_cut_row_tiles_of_page_strided_weights_stay_small():
+    """257 rows and more whose 128 x 64 tiles fit one round take them, but on
+    (N, K) weights with rows a multiple of 4 KB apart only in whole row tiles."""
+    L = _lib.lib()
+    geos = bi.geometries()
+    pick = lambda M, N, K, tb: geos[L.bi_gemm_pick_geometry(M, N, K, _lib.BF16, tb)]
+    small, large = (64, 64, 8), (128, 64, 4)
+    for M, N, K in ((257, 4096, 4096), (1500, 1024, 4096), (600, 2048, 6144), (450, 4096, 14336)):
+        assert pick(M, N, K, 1) == small, (M, N, K)
+        assert pick(M, N, K, 0) == large, (M, N, K)
+    for M, N, K in ((512, 4096, 4096), (1024, 2048, 6144), (257, 4096, 11008), (600, 2048, 2048)):
+        assert pick(M, N, K, 1) == pick(M, N, K, 0) == large, (M, N, K)
+
+
 def test_wide_tiles_are_not_picked_past_their_panel_limit():
     """A tile's rows of A must fit a 2 GiB buffer resource: K = 2^23 16-bit
     elements pass it in 128 rows and not in 64, so more than 256 rows keep the
     64 x 64 footprint there."""
     L = _lib.lib()
     geos = bi.geometries()
-    dense = lambda K: geos[L.bi_gemm_pick_geometry(300, 4096, K, _lib.BF16, 1)]
+    dense = lambda K: geos[L.bi_gemm_pick_geometry(384, 4096, K, _lib.BF16, 1)]
     assert dense((1 << 23) - 8) == (128, 64, 4)
     assert dense(1 << 23) == (64, 64, 8)
     quant = lambda K: geos[L.bi_qgemm_pick_geometry(1024, 11008, K, 4)]
