@@ -191,9 +191,10 @@ int pick_qgeometry(int64_t M, int64_t N, int64_t K, int bits, int group) {
   // one workgroup alone on a CU). Group 64: M = 1024, N = 11008 188 us in 64 x
   // 64 tiles, 162 in 128 x 64; M = 512, N = 4096 40 and 46; M = 2048, N = 4096
   // 140 and 120. Group 32: M = 1024, N = 11008 256 and 215. Group 128: 174 and
-  // 175, N = 32000 492 and 465.
-  const int64_t small = group == 32 ? 233 : group == 64 ? 173 : 158;
-  const int64_t large = group == 32 ? 355 : group == 64 ? 280 : 295;
+  // 175, N = 32000 492 and 465; its 8-bit codes cost the small tiles more (M =
+  // 800, N = 32000 452 and 401; M = 1024, N = 11008 202 and 176).
+  const int64_t small = group == 32 ? 233 : group == 64 ? 173 : bits == 8 ? 183 : 158;
+  const int64_t large = group == 32 ? 355 : group == 64 ? 280 : bits == 8 ? 290 : 295;
   const int64_t first = group == 32 ? 590 : 465;
   const int64_t t_small = std::max<int64_t>(ceil_div(t64, 256), 2) * small;
   const int64_t n_large = ceil_div(ceil_div(M, 128) * ceil_div(N, 64), 256);

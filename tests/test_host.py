@@ -127,13 +127,16 @@ def test_quantized_footprint_policy():
 
 def test_quantized_footprint_by_group_size():
     """More than 256 rows: 64 x 64 or 128 x 64 tiles by rounds of workgroups
-    whose times depend on the group size (M = 1024, N = 11008: 128 x 64 for
-    groups of 32 and 64 only). bi_qgemm_pick_geometry answers for 64."""
+    whose times depend on the group size and, for groups of 128, the code
+    width (M = 1024, N = 11008: 64 x 64 for 4-bit groups of 128 only).
+    bi_qgemm_pick_geometry answers for 64."""
     L = _lib.lib()
     geos = bi.geometries()
     pick = lambda M, N, gs, bits=4: geos[L.bi_qgemm_pick_group_geometry(M, N, 4096, gs, bits)]
     small, large = (64, 64, 8), (128, 64, 4)
     assert [pick(1024, 11008, gs) for gs in (32, 64, 128)] == [large, large, small]
+    assert pick(1024, 11008, 128, 2) == small
+    assert pick(1024, 11008, 128, 8) == pick(800, 32000, 128, 8) == large
     assert [pick(512, 4096, gs) for gs in (32, 64, 128)] == [small, small, small]
     assert [pick(1024, 32000, gs) for gs in (32, 64, 128)] == [large, large, large]
     for bits in (2, 4, 8):
