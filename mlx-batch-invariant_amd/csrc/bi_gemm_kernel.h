@@ -237,41 +237,54 @@ __device__ __forceinline__ uint4 load_any(const T* p) {
 // others zero; valid <= 0 gives zeros. A chunk that would run past the array
 // is read from the array's last 16 bytes and shifted.
 template <typename T>
-__device__ inline uint4 tail_chunk(const T* base, int64_t f, int64_t total, int64_t valid) {
-  constexpr int E = 16 / sizeof(T), W = 8 * sizeof(T);  // elements per chunk, bits per element
-  using Bits = typename std::conditional<sizeof(T) == 2, uint16_t, uint32_t>::type;
-  if (valid <= 0) return make_uint4(0, 0, 0, 0);
-  const int keep = valid < E ? (int)valid : E;
-  uint64_t lo = 0, hi = 0;
-  if (total >= E) {
-    const int64_t at = f < total - E ? f : total - E;
-    const uint4 v = load_any<T>(base + at);
-    lo = ((uint64_t)v.y << 32) | v.x;
-    hi = ((uint64_t)v.w << 32) | v.z;
-    int drop = (int)(f - at) * W;  // drop + keep * W <= 128
-    if (drop >= 64) {
-      lo = hi;
-      hi = 0;
-      drop -= 64;
-    }
-    if (drop) {
-      lo = (lo >> drop) | (hi << (64 - drop));
-      hi >>= drop;
-    }
-  } else {
+__device__ inline uint4 tail_chunk(const T* base, int64_t f, int64_t total, int valid) {
+  constexpr int E = 16 / sizeof(T);  // elements per chunk
+  if constexpr (sizeof(T) == 4) {  // four loads take less than the shifts
+    uint32_t w[4];
 #pragma unroll
-    for (int i = 0; i < E; i++) {
-      if (i < keep) {
-        const uint64_t e = __builtin_bit_cast(Bits, base[f + i]);
-        if (i < E / 2) lo |= e << (W * i);
-        else hi |= e << (W * (i - E / 2));
+    for (int i = 0; i < 4; i++) w[i] = i < valid ? __float_as_uint(base[f + i]) : 0u;
+    return make_uint4(w[0], w[1], w[2], w[3]);
+  } else {
+    if (valid <= 0) return make_uint4(0, 0, 0, 0);
+    const int keep = valid < E ? valid : E;
+    uint4 v = make_uint4(0, 0, 0, 0);
+    if (total >= E) {
+      const int64_t over = f - (total - E);
+      const int drop = over > 0 ? (int)over : 0;  // drop + keep <= E
+      v = load_any<T>(base + f - drop);
+      if (drop) {  // (the array's last chunks alone)
+        uint64_t lo = ((uint64_t)v.y << 32) | v.x, hi = ((uint64_t)v.w << 32) | v.z;
+        int bits = drop * 16;
+        if (bits >= 64) {
+          lo = hi;
+          hi = 0;
+          bits -= 64;
+        }
+        if (bits) {
+          lo = (lo >> bits) | (hi << (64 - bits));
+          hi >>= bits;
+        }
+        v = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
       }
+    } else {
+      uint32_t w[4] = {0, 0, 0, 0};
+#pragma unroll
+      for (int i = 0; i < E; i++)
+        if (i < keep)
+          w[i / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, base[f + i]) << (16 * (i & 1));
+      v = make_uint4(w[0], w[1], w[2], w[3]);
     }
+    if (keep < E) {  // (a row's last chunk alone)
+      uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int left = keep - 2 * i;  // elements of this word
+        w[i] = left >= 2 ? w[i] : left <= 0 ? 0u : w[i] & 0xFFFFu;
+      }
+      v = make_uint4(w[0], w[1], w[2], w[3]);
+    }
+    return v;
   }
-  const int bits = keep * W;
-  if (bits < 64) lo &= ((uint64_t)1 << bits) - 1;
-  hi &= bits <= 64 ? 0 : ~(uint64_t)0 >> (128 - bits);
-  return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
 }
 
 // Raw buffer resources (CDNA "V#"): loads whose byte offset is at or past
@@ -484,13 +497,14 @@ struct GemmTile {
   // (K, N) chunk past N reads on into the next rows: what they produce lies
   // outside C and is never stored. Stages that lie wholly below kfull() read
   // inside the operands with plain 16-byte loads; the rest go through
-  // tail_chunk, which zeroes elements past K. The waves that do not compute,
+  // tail_chunk, which zeroes elements past K (with nothing but a tail, K below
+  // a stage, a launch takes up to 0.4 us more than one element per load). The waves that do not compute,
   // where there are such, load and stage every operand, so a stage is written
   // while the one before it is computed. Bound by those loads: an access that
   // is not 16-byte aligned takes the address unit about 64 cycles a wave
   // instead of 16 (any smaller alignment alike), 0.5 us per 32 KB stage.
   // Against one element per load and two barriers a stage (bf16): M = 301,
-  // K = 1001, N = 3001 (K, N) 43.2 -> 13.7 us; M = 2048, K = 4095, N = 4096
+  // K = 1001, N = 3001 (K, N) 43.0 -> 12.8 us; M = 2048, K = 4095, N = 4096
   // (N, K) 938 -> 134 us; M = 1 55 -> 10.8 us.
   static constexpr int RNT = NW > CW ? 64 * (NW - CW) : NT;  // loading threads
   static constexpr int RLA = (A_CH + RNT - 1) / RNT, RLB = (B_CH + RNT - 1) / RNT;
@@ -508,20 +522,25 @@ struct GemmTile {
     return K - (EPC - 1 + N - 1) / N;
   }
 
+  // (Sizes are below 2^31, the host checks: one 32 x 32 bit product a pointer.)
+  static __device__ __forceinline__ int64_t times(int row, int64_t ld) {
+    return (int64_t)((uint64_t)(uint32_t)row * (uint32_t)ld);
+  }
   __device__ __forceinline__ void init_ragged() {
     rtid = tid - (NT - RNT);
+    const int m = (int)m0, n = (int)n0;
 #pragma unroll
     for (int i = 0; i < RLA; i++) {
       const int q = rtid + i * RNT;
-      rg_a[i] = A + min(m0 + q / RC, M - 1) * K + (q % RC) * EPC;
+      rg_a[i] = A + times(min(m + q / RC, (int)M - 1), K) + (q % RC) * EPC;
     }
 #pragma unroll
     for (int i = 0; i < RLB; i++) {
       const int q = rtid + i * RNT;
       if constexpr (TB)
-        rg_b[i] = B + min(n0 + q / RC, N - 1) * K + (q % RC) * EPC;
+        rg_b[i] = B + times(min(n + q / RC, (int)N - 1), K) + (q % RC) * EPC;
       else  // (the last loads of an uneven split lie past the tile: row 0)
-        rg_b[i] = B + (int64_t)(q < B_CH ? q / NN_CPR : 0) * N + min(n0 + (q % NN_CPR) * EPC, N - 1);
+        rg_b[i] = B + times(q < B_CH ? q / NN_CPR : 0, N) + min(n + (q % NN_CPR) * EPC, (int)N - 1);
     }
   }
 
@@ -534,23 +553,20 @@ struct GemmTile {
   }
 
   __device__ __forceinline__ void rg_load_tail(int64_t s, RStage& st) const {
-    const int64_t k0 = s * EPS;
+    const int64_t k0 = s * EPS, bo = TB ? k0 : k0 * N;
+    const int kleft = (int)(K - k0);
 #pragma unroll
-    for (int i = 0; i < RLA; i++) {
-      const int q = rtid + i * RNT;
-      const int64_t r = min(m0 + q / RC, M - 1), k = k0 + (q % RC) * EPC;
-      st.a[i] = tail_chunk<T>(A, r * K + k, M * K, K - k);
-    }
+    for (int i = 0; i < RLA; i++)
+      st.a[i] = tail_chunk<T>(A, rg_a[i] - A + k0, M * K, kleft - (rtid + i * RNT) % RC * EPC);
 #pragma unroll
     for (int i = 0; i < RLB; i++) {
       const int q = rtid + i * RNT;
-      if constexpr (TB) {
-        const int64_t r = min(n0 + q / RC, N - 1), k = k0 + (q % RC) * EPC;
-        st.b[i] = tail_chunk<T>(B, r * K + k, N * K, K - k);
-      } else {
-        const int64_t k = k0 + q / NN_CPR, n = n0 + (q % NN_CPR) * EPC;
-        st.b[i] = tail_chunk<T>(B, k * N + n, K * N, k < K ? N - n : 0);
-      }
+      if constexpr (TB)
+        st.b[i] = tail_chunk<T>(B, rg_b[i] - B + bo, N * K, kleft - q % RC * EPC);
+      else
+        st.b[i] = tail_chunk<T>(B, rg_b[i] - B + bo, K * N,
+                                (q < B_CH ? q / NN_CPR : 0) < kleft
+                                    ? (int)N - ((int)n0 + (q % NN_CPR) * EPC) : 0);
     }
   }
 
