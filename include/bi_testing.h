@@ -29,8 +29,9 @@ int bi_gemm_num_geometries(void);
 int bi_gemm_geometry_info(int g, int* block_m, int* block_n, int* waves);
 
 /* The geometry bi_gemm would launch for this problem with 16-byte aligned
- * operands (for others it replaces a footprint that takes aligned operands
- * only, the 256 x 128 one, by 128 x 128). */
+ * operands whose panels stay below 2 GiB (others take register-staged forms of
+ * the 16 x 16, 64 x 16, 64 x 32, 64 x 64 or 128 x 128 footprints, picked by a
+ * rule of their own that no entry point exposes). */
 int bi_gemm_pick_geometry(int64_t M, int64_t N, int64_t K, int dtype, int trans_b);
 
 /* bi_gemm with the geometry forced to `g` (same arguments and semantics);

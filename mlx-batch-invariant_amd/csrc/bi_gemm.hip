@@ -242,8 +242,8 @@ VecFlags vec_flags(const void* a, const void* b, int64_t N, int64_t K, int dtype
   return v;
 }
 
-// Geometry for operands that are not 16-byte aligned (the register-staged
-// kernels): the least estimated time per element of K, from a grid of every
+// Geometry for operands that are not 16-byte aligned, or whose panels pass 2 GiB
+// (the register-staged kernels): the least estimated time per element of K, from a grid of every
 // footprint that has such a kernel over M = 1..1024, K = 501..4095 and N =
 // 601..5001 (both layouts, bf16 and fp32; every size odd). A 64 x 32, 64 x 64
 // or 128 x 128 tile costs a round of the CUs each time its tiles pass a

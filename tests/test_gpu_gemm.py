@@ -168,7 +168,7 @@ def test_large_footprints_agree(cuda, trans_b):
 def test_unaligned_operands_leave_the_aligned_only_footprint(cuda):
     """The 256x128 footprint (its loading waves issue every load) takes
     16-byte aligned operands only: forcing it on others raises, and bi_gemm
-    launches the 128x128 footprint instead. Misaligned bases and a K that is
+    launches a register-staged footprint instead. Misaligned bases and a K that is
     not a multiple of 8 give the bits of the same values in aligned storage
     and of every footprint that takes them."""
     from mlx_batch_invariant import _lib
@@ -241,6 +241,25 @@ def test_ragged_operands(cuda, trans_b, M, K, N):
                 dname, "picked" if gi is None else geos[gi], int((~same).sum()))
             assert not bool(got[:max(1, M - 1), :max(1, N - 1)].isnan().any())
         assert ran == 6
+
+
+def test_weight_of_two_gib_and_more(cuda):
+    """An aligned (K, N) weight past the 2 GiB of a buffer resource takes the
+    register-staged kernels with 64-bit offsets: its first, middle and last
+    columns have the bits of the same columns in a weight of their own."""
+    M, K, N = 3, 4104, 262400
+    assert K * N * 2 > 1 << 31 and N % 8 == 0
+    a = rn((M, K), torch.bfloat16, 71, device=cuda)
+    g = torch.Generator(device=cuda).manual_seed(72)
+    w = torch.empty(K, N, dtype=torch.bfloat16, device=cuda).normal_(0.0, K ** -0.5, generator=g)
+    try:
+        y = bi.matmul(a, w)
+        for n in (0, 131072 - 32, N - 64):
+            want = bi.matmul(a, w[:, n:n + 64].contiguous())
+            assert ndiff(y[:, n:n + 64].contiguous(), want) == 0, n
+    finally:
+        del w
+        torch.cuda.empty_cache()
 
 
 def test_kn_and_nk_layouts_agree(cuda):
