@@ -485,7 +485,7 @@ bool scored_fits(int64_t N, int64_t vs2, int esz) {
 // where the walk along the keys is what takes the time and the grid leaves
 // compute units idle (one query row of one sequence, 32/8 heads, N = 8192,
 // keys and values in the last-level cache: D = 256 118 -> 28 us, D = 128
-// 26.0 -> 20.7, with an array mask 48 -> 28; in HBM 122 -> 41, 53 -> 31, 72 ->
+// 26.0 -> 20.7, with an array mask 67 -> 38; in HBM 122 -> 41, 53 -> 31, 72 ->
 // 41), and not where a second launch and the scores' way through memory cost
 // more (8 sequences, D = 128: 41 and 50 us).
 // Both times, in microseconds, by least squares over a grid of H/Hkv = 32/8,
